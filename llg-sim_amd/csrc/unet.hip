@@ -275,154 +275,175 @@ __global__ __launch_bounds__(256) void k_conv3x3_tile(const uint16_t *__restrict
     }
 }
 
-// Weight gradient: dw[tap][co][ci] += sum_p dz[p][co] * x[p + off(tap)][ci].
-// Block = 4 waves over one tap and one (16*MT) x (16*NT) tile and a pixel
-// chunk, taken kSlice pixels at a time: the block loads 4-pixel x 4-channel
-// blocks of dz and of the shifted x (four 8-byte loads each), transposes
-// them in registers into LDS tiles [channel][pixel], and each wave multiplies
-// its quarter of the slice in 16-pixel MFMA steps (8-byte LDS reads of 4
-// consecutive pixels).
-// The waves' partial tiles are summed through LDS and added to dw with FP32
-// atomics.
+// Weight and bias gradient: dw[tap][co][ci] = sum_p dz[p][co] x[p + off(tap)][ci],
+// db[co] = sum_p dz[p][co].  The reduction runs over pixels, which a matrix-core
+// operand wants eight at a time per channel while memory holds channels
+// together: the tiles are staged in LDS as they lie in memory ([pixel][channel])
+// and read with the transposing LDS read (ds_read_b64_tr_b16, four pixels of
+// one channel per lane), so a tap is an address offset and needs no copy of its
+// own.  A block takes one (16*MT) x (16*NT) channel tile and a contiguous run
+// of 16 x 16 pixel tiles: per tile dz and x with its one-pixel halo are loaded
+// once (the next tile's loads are in flight during the products) and serve all
+// nine taps, whose 9*MT*NT partial tiles stay in registers until the run ends.
+// Each wave takes four pixel rows (two K = 32 products of two 16-pixel rows);
+// the waves' sums are added through LDS and written to the block's own row of
+// `part`, which k_part_sum reduces: no atomics, so gradients do not depend on
+// the order in which blocks finish.  The bias gradient is one more product,
+// with ones, in the blocks of the first ci tile.
+// Bound by the tiles' loads where a layer has few channels (32 x 32: 288
+// multiply-adds per byte) and by LDS reads elsewhere.  Against one block per tap
+// with 8-byte loads and atomics (and a pass of its own for the bias): 11.3 -> 1.3 ms for the fifteen layers of a
+// 8 x 528 x 528 step (742 -> 84 us per 32 x 32 tiled layer).
+constexpr int kWgT = 16, kWgX = kWgT + 2;   // pixel tile and tile with halo
 template <int MT, int NT>
-__global__ __launch_bounds__(256) void k_conv3x3_wgrad(const uint16_t *__restrict__ dz, int cout,
-                                                       const uint16_t *__restrict__ x, int xs, int xo, int cin,
-                                                       float *__restrict__ dw, int B, int H, int W, int chunk) {
-    constexpr int kSlice = 64;          // pixels per LDS fill
-    constexpr int kRow = kSlice + 4;    // LDS row stride (elements) of the transposed tiles
-    __shared__ __align__(16) uint16_t sa[16 * MT][kRow];   // dz^T: [co][pixel]
-    __shared__ __align__(16) uint16_t sb[16 * NT][kRow];   // x^T:  [ci][pixel]
-    __shared__ f32x4 red[4][MT * NT][64];
-    const int P = B * H * W;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int li = lane & 15, lk = (lane >> 4) * 4;
-    const int tap = blockIdx.z, dy = tap / 3 - 1, dx = tap % 3 - 1;
-    const int co_tiles = cout / (16 * MT);
-    const int co_base = (blockIdx.y % co_tiles) * 16 * MT;
-    const int ci_base = (blockIdx.y / co_tiles) * 16 * NT;
-    const int p_begin = blockIdx.x * chunk;
-    const int p_end = min(P, p_begin + chunk);
-    constexpr int nA = kSlice / 4 * 4 * MT, nB = kSlice / 4 * 4 * NT;   // (pixel quad, channel quad) items
-    f32x4 acc[MT][NT];
+__global__ __launch_bounds__(256, 2) void k_conv3x3_wgrad(const uint16_t *__restrict__ dz, int cout,
+                                                          const uint16_t *__restrict__ x, int xs, int xo, int cin,
+                                                          float *__restrict__ part, int B, int H, int W) {
+    constexpr int CO = 16 * MT, CI = 16 * NT;
+    constexpr int NX = kWgX * kWgX * (CI / 8), NZ = kWgT * kWgT * (CO / 8);   // 16-byte pieces of a tile
+    constexpr int LX = (NX + 255) / 256, LZ = (NZ + 255) / 256;
+    constexpr size_t kStage = 16 * (size_t)(NX + NZ), kRed = sizeof(f32x4) * 4 * MT * NT * 64;
+    __shared__ __align__(16) unsigned char smem[kStage > kRed ? kStage : kRed];
+    uint16_t *xin = reinterpret_cast<uint16_t *>(smem);      // [kWgX * kWgX][CI]
+    uint16_t *zin = xin + kWgX * kWgX * CI;                  // [kWgT * kWgT][CO]
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4, j = lane & 15;
+    const int co_tiles = cout / CO;
+    const int co_base = ((int)blockIdx.y % co_tiles) * CO, ci_base = ((int)blockIdx.y / co_tiles) * CI;
+    const int ntx = (W + kWgT - 1) / kWgT, nty = (H + kWgT - 1) / kWgT, ntile = ntx * nty * B;
+    const int t0 = (int)((int64_t)ntile * blockIdx.x / gridDim.x),
+              t1 = (int)((int64_t)ntile * (blockIdx.x + 1) / gridDim.x);
+    f32x4 acc[9][MT][NT], accb[MT];
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
+    for (int mt = 0; mt < MT; ++mt) {
+        accb[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int p0 = p_begin; p0 < p_end; p0 += kSlice) {
-        __syncthreads();   // the previous slice's reads are done
-        for (int e = threadIdx.x; e < nA + nB; e += 256) {
-            const bool isA = e < nA;
-            const int f = isA ? e : e - nA;
-            const int cq = f % (isA ? 4 * MT : 4 * NT), pq = f / (isA ? 4 * MT : 4 * NT);
-            bf16x4 v[4];
-            const int pb = p0 + pq * 4;
-            int xc = pb % W, yc = (pb / W) % H;   // column and row of pixel pb, advanced below
+        for (int tap = 0; tap < 9; ++tap)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int p = pb + r;
-                v[r] = bf16x4{0, 0, 0, 0};
-                if (p < p_end) {
-                    if (isA) {
-                        v[r] = *(const bf16x4 *)(dz + (int64_t)p * cout + co_base + cq * 4);
-                    } else {
-                        const int xx = xc + dx, yy = yc + dy;
-                        if (xx >= 0 && xx < W && yy >= 0 && yy < H) {
-                            const int64_t q = (int64_t)p + dy * W + dx;
-                            v[r] = *(const bf16x4 *)(x + q * xs + xo + ci_base + cq * 4);
-                        }
-                    }
-                }
-                if (++xc == W) {   // next pixel starts a new row (and perhaps a new batch image)
-                    xc = 0;
-                    if (++yc == H) yc = 0;
-                }
-            }
-            uint16_t(*t)[kRow] = isA ? sa : sb;
+            for (int nt = 0; nt < NT; ++nt) acc[tap][mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    uint4 rx[LX], rz[LZ];
+    auto fetch = [&](int t) {
+        const int tx = t % ntx, ty = (t / ntx) % nty, b = t / (ntx * nty);
+        const int x0 = tx * kWgT, y0 = ty * kWgT;
 #pragma unroll
-            for (int c = 0; c < 4; ++c)
-                *(bf16x4 *)&t[cq * 4 + c][pq * 4] = bf16x4{v[0][c], v[1][c], v[2][c], v[3][c]};
+        for (int k = 0; k < LX; ++k) {
+            const int e = threadIdx.x + k * 256, pix = e / (CI / 8), c = (e % (CI / 8)) * 8;
+            const int yy = y0 + pix / kWgX - 1, xx = x0 + pix % kWgX - 1;
+            rx[k] = uint4{0u, 0u, 0u, 0u};
+            if (e < NX && yy >= 0 && yy < H && xx >= 0 && xx < W)
+                rx[k] = *reinterpret_cast<const uint4 *>(x + ((int64_t)(b * H + yy) * W + xx) * xs + xo + ci_base + c);
         }
+#pragma unroll
+        for (int k = 0; k < LZ; ++k) {
+            const int e = threadIdx.x + k * 256, pix = e / (CO / 8), c = (e % (CO / 8)) * 8;
+            const int yy = y0 + pix / kWgT, xx = x0 + pix % kWgT;
+            rz[k] = uint4{0u, 0u, 0u, 0u};
+            if (e < NZ && yy < H && xx < W)
+                rz[k] = *reinterpret_cast<const uint4 *>(dz + ((int64_t)(b * H + yy) * W + xx) * cout + co_base + c);
+        }
+    };
+    // eight pixels (k = 8 g + 0..7) of channel j of the 16 at p
+    auto frag = [&](const uint16_t *p, int row_len) -> bf16x8 {
+        typedef __attribute__((address_space(3))) bf16x4 *lds4;
+        const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)p);
+        const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)(p + 4 * row_len));
+        typedef short s16x8 __attribute__((ext_vector_type(8)));
+        return __builtin_bit_cast(bf16x8, (s16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+    };
+    const __bf16 one = (__bf16)1.0f;
+    const bf16x8 ones = {one, one, one, one, one, one, one, one};
+    if (t0 < t1) fetch(t0);
+    for (int t = t0; t < t1; ++t) {
+        __syncthreads();   // the previous tile's reads are done
+#pragma unroll
+        for (int k = 0; k < LX; ++k)
+            if (threadIdx.x + k * 256 < NX) reinterpret_cast<uint4 *>(xin)[threadIdx.x + k * 256] = rx[k];
+#pragma unroll
+        for (int k = 0; k < LZ; ++k)
+            if (threadIdx.x + k * 256 < NZ) reinterpret_cast<uint4 *>(zin)[threadIdx.x + k * 256] = rz[k];
+        __syncthreads();
+        if (t + 1 < t1) fetch(t + 1);
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            // lane group g: row g / 2 of the step's two, columns 8 (g % 2) ..
+            const int row = (wave * 2 + s) * 2 + (g >> 1), col = (g & 1) * 8 + (j >> 2);
+            const uint16_t *za = zin + (row * kWgT + col) * CO + (j & 3) * 4;
+            const uint16_t *xa = xin + (row * kWgX + col) * CI + (j & 3) * 4;
+            bf16x8 a[MT];
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) a[mt] = frag(za + mt * 16, CO);
+            if (ci_base == 0) {
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt)
+                    accb[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[mt], ones, accb[mt], 0, 0, 0);
+            }
+#pragma unroll
+            for (int tap = 0; tap < 9; ++tap) {
+                bf16x8 bx[NT];
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt) bx[nt] = frag(xa + ((tap / 3) * kWgX + tap % 3) * CI + nt * 16, CI);
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                    for (int nt = 0; nt < NT; ++nt)
+                        acc[tap][mt][nt] =
+                            __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[mt], bx[nt], acc[tap][mt][nt], 0, 0, 0);
+            }
+        }
+    }
+    // the four waves' sums through LDS, one tap at a time; lane holds rows
+    // 4 (lane / 16) + r (co), column lane % 16 (ci) of every 16 x 16 tile
+    f32x4(*red)[MT * NT][64] = reinterpret_cast<f32x4(*)[MT * NT][64]>(smem);
+    float *out = part + (int64_t)blockIdx.x * ((int64_t)9 * cout * cin + cout);
+#pragma unroll
+    for (int tap = 0; tap < 9; ++tap) {
         __syncthreads();
 #pragma unroll
-        for (int ks = 0; ks < kSlice / 64; ++ks) {
-            const int kp = wave * (kSlice / 4) + ks * 16 + lk;   // this lane's 4 consecutive pixels
-            bf16x4 a[MT], b[NT];
+        for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-            for (int mt = 0; mt < MT; ++mt) a[mt] = *(const bf16x4 *)&sa[mt * 16 + li][kp];
+            for (int nt = 0; nt < NT; ++nt) red[wave][mt * NT + nt][lane] = acc[tap][mt][nt];
+        __syncthreads();
+        for (int e = threadIdx.x; e < MT * NT * 64; e += 256) {
+            const int t = e / 64, ln = e % 64;
+            const f32x4 sum = red[0][t][ln] + red[1][t][ln] + red[2][t][ln] + red[3][t][ln];
+            const int ci = ci_base + (t % NT) * 16 + (ln & 15);
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt) b[nt] = *(const bf16x4 *)&sb[nt * 16 + li][kp];
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-                for (int nt = 0; nt < NT; ++nt)
-                    acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[mt], b[nt], acc[mt][nt], 0, 0, 0);
+            for (int r = 0; r < 4; ++r) {
+                const int co = co_base + (t / NT) * 16 + (ln >> 4) * 4 + r;
+                out[((int64_t)tap * cout + co) * cin + ci] = sum[r];
+            }
         }
     }
+    if (ci_base == 0) {   // uniform over the block
+        __syncthreads();
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
+        for (int mt = 0; mt < MT; ++mt) red[wave][mt][lane] = accb[mt];
+        __syncthreads();
+        for (int e = threadIdx.x; e < MT * 64; e += 256) {
+            const int t = e / 64, ln = e % 64;
+            if (ln & 15) continue;   // every column of the product with ones is the same sum
+            const f32x4 sum = red[0][t][ln] + red[1][t][ln] + red[2][t][ln] + red[3][t][ln];
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) red[wave][mt * NT + nt][lane] = acc[mt][nt];
-    __syncthreads();
-    // thread t sums entry (tile t/64, lane t%64) of the four waves
-    for (int e = threadIdx.x; e < MT * NT * 64; e += 256) {
-        const int t = e / 64, ln = e % 64;
-        const f32x4 sum = red[0][t][ln] + red[1][t][ln] + red[2][t][ln] + red[3][t][ln];
-        const int mt = t / NT, nt = t % NT;
-        const int ci = ci_base + nt * 16 + (ln & 15);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int co = co_base + mt * 16 + (ln >> 4) * 4 + r;
-            atomicAdd(dw + ((int64_t)tap * cout + co) * cin + ci, sum[r]);
+            for (int r = 0; r < 4; ++r) out[(int64_t)9 * cout * cin + co_base + t * 16 + (ln >> 4) * 4 + r] = sum[r];
         }
     }
 }
 
-// db[c] += sum over the block's pixel chunk of dz[p][c] (cout <= 256): the
-// 256 threads form G = 256 / cout groups of cout channel lanes; group g sums
-// pixels p0 + g, p0 + g + G, ...; the groups are reduced through LDS.
-__global__ __launch_bounds__(256) void k_bias_grad(const uint16_t *__restrict__ dz, int cout, int P, int chunk,
-                                                   float *__restrict__ db) {
-    __shared__ float part[256];
-    const int G = 256 / cout;
-    const int t = threadIdx.x, g = t / cout, c = t % cout;
-    const int p0 = blockIdx.x * chunk, p1 = min(P, p0 + chunk);
+// out[i] = sum of part[s][i] over the nrow rows of length n: four row groups of
+// 64 columns per block, added through LDS
+__global__ __launch_bounds__(256) void k_part_sum(const float *__restrict__ part, int nrow, int64_t n,
+                                                  float *__restrict__ out) {
+    __shared__ float red[4][64];
+    const int c = threadIdx.x & 63, g = threadIdx.x >> 6;
+    const int64_t i = (int64_t)blockIdx.x * 64 + c;
     float s = 0.f;
-    if (g < G)
-        for (int p = p0 + g; p < p1; p += G) s += bf2f(dz[(int64_t)p * cout + c]);
-    part[t] = s;
-    __syncthreads();
-    if (t < cout) {
-        float r = 0.f;
-        for (int k = 0; k < G; ++k) r += part[k * cout + t];
-        atomicAdd(db + t, r);
+    if (i < n) {
+#pragma unroll 8
+        for (int r = g; r < nrow; r += 4) s += part[(int64_t)r * n + i];
     }
-}
-
-// k_bias_grad eight channels (16 bytes) per thread: cout a multiple of 8 and
-// at most 256 (groups of 8 channels per thread, pixel lanes over the rest)
-__global__ __launch_bounds__(256) void k_bias_grad_v8(const uint16_t *__restrict__ dz, int cout, int P, int chunk,
-                                                      float *__restrict__ db) {
-    __shared__ float part[256 * 8];
-    const int C8 = cout / 8, G = 256 / C8;
-    const int t = threadIdx.x, g = t / C8, c8 = t - g * C8;
-    const int p0 = blockIdx.x * chunk, p1 = min(P, p0 + chunk);
-    float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (g < G)
-        for (int p = p0 + g; p < p1; p += G) {
-            const uint4 q = *reinterpret_cast<const uint4 *>(dz + (int64_t)p * cout + c8 * 8);
-            const uint16_t *h = reinterpret_cast<const uint16_t *>(&q);
-#pragma unroll
-            for (int k = 0; k < 8; ++k) s[k] += bf2f(h[k]);
-        }
-#pragma unroll
-    for (int k = 0; k < 8; ++k) part[t * 8 + k] = g < G ? s[k] : 0.f;
+    red[g][c] = s;
     __syncthreads();
-    if (t < cout) {
-        const int cg = t / 8, ck = t - cg * 8;
-        float r = 0.f;
-        for (int k = 0; k < G; ++k) r += part[(k * C8 + cg) * 8 + ck];
-        atomicAdd(db + t, r);
-    }
+    if (g == 0 && i < n) out[i] = (red[0][c] + red[1][c]) + (red[2][c] + red[3][c]);
 }
 
 // 2x2 average pool of a slice: y[b][Y][X][c] = mean of x[b][2Y+i][2X+j][xo+c]
@@ -692,6 +713,7 @@ struct UNet {
     int64_t nparam = 0;
     float *d_p = nullptr, *d_g = nullptr, *d_m = nullptr, *d_v = nullptr;
     uint16_t *d_wbf = nullptr;    // bf16 forward and transposed weights of every conv
+    float *d_part = nullptr;      // partial weight gradients of one layer
     int64_t t = 0;                // Adam step count
     double *d_loss = nullptr, *h_loss = nullptr;
     std::vector<void *> bufs;
@@ -756,6 +778,11 @@ struct UNet {
                 cv.wb = d_wbf + o;
                 o += (int64_t)9 * cv.cin * cv.cout;
             }
+            int64_t npart = 0;
+            for (size_t k = 0; k < conv.size(); ++k)
+                npart = std::max(npart, wgrad_split(conv[k].cout, conv[k].cin, level_of((int)k)) *
+                                            ((int64_t)9 * conv[k].cin * conv[k].cout + conv[k].cout));
+            d_part = dalloc<float>(npart);
             d_loss = dalloc<double>(1);
             LLGMI_HIP(hipHostMalloc((void **)&h_loss, sizeof(double), hipHostMallocDefault));
             // activations and gradients
@@ -923,43 +950,38 @@ struct UNet {
     void wgrad(const uint16_t *dzp, int co, const uint16_t *x, int xs, int xo, int ci, const UNetConv &cv, int l) {
         if (co % 16 || ci % 16 || xo + ci > xs || co != cv.cout || ci != cv.cin)
             throw Error(LLGMI_ERR_INVALID, "internal: weight-gradient shape");
-        const int64_t P = pl(l);
-        float *dw = d_g + cv.w_off;
-        const int mt = (co / 16) % 2 == 0 ? 2 : 1, nt = (ci / 16) % 2 == 0 ? 2 : 1;
-        // pixel chunk per block: about 2048 blocks in all (each block ends in
-        // 16*mt x 16*nt x 4 atomics), at least 2048 pixels, a multiple of 64
-        const int tiles = (co / (16 * mt)) * (ci / (16 * nt));
-        const int64_t nchunks = std::max<int64_t>(1, 2048 / (9 * tiles));
-        const int chunk = (int)std::max<int64_t>(2048, ((P + nchunks - 1) / nchunks + 63) / 64 * 64);
-        const int gx = (int)((P + chunk - 1) / chunk);
-        const dim3 grid(gx, tiles, 9);
-        if (mt == 2 && nt == 2)
-            hipLaunchKernelGGL((k_conv3x3_wgrad<2, 2>), grid, dim3(256), 0, stream, dzp, co, x, xs, xo, ci, dw, B,
-                               hl(l), wl(l), chunk);
-        else if (mt == 2)
-            hipLaunchKernelGGL((k_conv3x3_wgrad<2, 1>), grid, dim3(256), 0, stream, dzp, co, x, xs, xo, ci, dw, B,
-                               hl(l), wl(l), chunk);
-        else if (nt == 2)
-            hipLaunchKernelGGL((k_conv3x3_wgrad<1, 2>), grid, dim3(256), 0, stream, dzp, co, x, xs, xo, ci, dw, B,
-                               hl(l), wl(l), chunk);
-        else
-            hipLaunchKernelGGL((k_conv3x3_wgrad<1, 1>), grid, dim3(256), 0, stream, dzp, co, x, xs, xo, ci, dw, B,
-                               hl(l), wl(l), chunk);
-        const int bchunk = 1024;
-        if (co > 256) throw Error(LLGMI_ERR_INVALID, "internal: bias gradient over 256 channels");
-        if (co % 8 == 0)
-            hipLaunchKernelGGL(k_bias_grad_v8, dim3((unsigned)((P + bchunk - 1) / bchunk)), dim3(256), 0, stream, dzp,
-                               co, (int)P, bchunk, d_g + cv.b_off);
-        else
-            hipLaunchKernelGGL(k_bias_grad, dim3((unsigned)((P + bchunk - 1) / bchunk)), dim3(256), 0, stream, dzp,
-                               co, (int)P, bchunk, d_g + cv.b_off);
+        const int mt = wgrad_mt(co), nt = wgrad_nt(co, ci);
+        const dim3 grid((unsigned)wgrad_split(co, ci, l), (unsigned)((co / (16 * mt)) * (ci / (16 * nt))));
+        auto go = [&](auto kern) {
+            hipLaunchKernelGGL(kern, grid, dim3(256), 0, stream, dzp, co, x, xs, xo, ci, d_part, B, hl(l), wl(l));
+        };
+        if (mt == 3) go(k_conv3x3_wgrad<3, 1>);
+        else if (mt == 2) nt == 2 ? go(k_conv3x3_wgrad<2, 2>) : go(k_conv3x3_wgrad<2, 1>);
+        else nt == 2 ? go(k_conv3x3_wgrad<1, 2>) : go(k_conv3x3_wgrad<1, 1>);
+        // a layer's weights and bias are consecutive in the parameter vector
+        const int64_t n = (int64_t)9 * co * ci + co;
+        hipLaunchKernelGGL(k_part_sum, dim3((unsigned)((n + 63) / 64)), dim3(256), 0, stream, d_part, (int)grid.x, n,
+                           d_g + cv.w_off);
         LLGMI_LAUNCH_CHECK();
+    }
+    // channel tiles of the weight gradient (48 output channels in one tile of
+    // three, then with one input tile: three by two spill) and the pixel runs a layer is split into: two blocks per CU in all,
+    // no more than there are pixel tiles, a multiple of the eight XCDs so that
+    // the channel tiles of one run share an L2
+    static int wgrad_mt(int co) { return co % 32 == 0 ? 2 : co % 48 == 0 ? 3 : 1; }
+    static int wgrad_nt(int co, int ci) { return wgrad_mt(co) < 3 && ci % 32 == 0 ? 2 : 1; }
+    int wgrad_split(int co, int ci, int l) const {
+        const int64_t tiles = (int64_t)B * ((hl(l) + kWgT - 1) / kWgT) * ((wl(l) + kWgT - 1) / kWgT);
+        int64_t s = std::max<int64_t>(1, 512 / ((co / (16 * wgrad_mt(co))) * (ci / (16 * wgrad_nt(co, ci)))));
+        if (s > 8) s -= s % 8;
+        return (int)std::min(s, tiles);
     }
 
     // conv index: enc l -> 2l, 2l+1; dec l (2..0) -> 8 + 2(2-l), +1; head -> 14
     const UNetConv &enc(int l, int k) const { return conv[(size_t)(2 * l + k)]; }
     const UNetConv &dec(int l, int k) const { return conv[(size_t)(2 * kLevels + 2 * (kLevels - 2 - l) + k)]; }
     const UNetConv &head() const { return conv.back(); }
+    static int level_of(int k) { return k < 2 * kLevels ? k / 2 : k == 4 * kLevels - 2 ? 0 : kLevels - 2 - (k - 2 * kLevels) / 2; }
 
     void forward(const uint16_t *x) {
         for (int l = 0; l < kLevels; ++l) {
@@ -1009,7 +1031,6 @@ struct UNet {
     // gradient of the loss w.r.t. every parameter into d_g (overwritten)
     double loss_grad(const uint16_t *x, const uint16_t *tgt) {
         forward(x);
-        LLGMI_HIP(hipMemsetAsync(d_g, 0, sizeof(float) * (size_t)nparam, stream));
         LLGMI_HIP(hipMemsetAsync(d_loss, 0, sizeof(double), stream));
         const double count = (double)B * std::min(wv, W) * std::min(hv, H) * cout_real;
         hipLaunchKernelGGL(k_mse, dim3(grid_of(pl(0) * cout)), dim3(kNT), 0, stream, out, tgt, cout, cout_real, wv,

@@ -92,6 +92,35 @@ def test_gradients_match_oracle(gpu_lib, tile, monkeypatch):
     assert tot <= 3e-4
 
 
+# Planes smaller than one 16 x 16 pixel tile of the weight gradient, with
+# remainder rows and columns of tiles and with several runs per layer; channel
+# tiles of 16, 32 and 48.  On so few pixels one bf16 rounding that falls the
+# other way (2^-9 of an activation) shows in every layer before it, so the bar
+# is accuracy: the device and the bf16 emulation are two roundings of one
+# network, and the device's distance from float64 may not exceed twice the
+# emulation's per tensor (a dropped pixel row or channel is an error of order
+# 1 / 16 or more against 1e-2).
+@pytest.mark.parametrize("batch,height,width,base,out", [
+    (1, 8, 8, 16, 3), (3, 16, 16, 32, 36), (1, 24, 40, 32, 36), (2, 40, 24, 16, 40), (1, 72, 8, 32, 16)])
+def test_gradient_tile_edges(gpu_lib, batch, height, width, base, out):
+    s = U.Shape(batch=batch, height=height, width=width, out_channels=out, base=base, valid_width=width - 1,
+                valid_height=height - 3)
+    net, p, x, t, xd, td = _setup(gpu_lib, s, 11 + height)
+    loss = net.loss_grad(xd, td)
+    g = net.get_grads().astype(np.float64)
+    again = net.loss_grad(xd, td)
+    loss_o, g_o, _ = U.loss_and_grad(s, p, x, t, bf16=True)
+    _, g_64, _ = U.loss_and_grad(s, p, x, t, bf16=False)
+    assert abs(loss - loss_o) <= 1e-3 * loss_o and abs(again - loss) <= 1e-12 * loss
+    assert np.array_equal(net.get_grads(), g.astype(np.float32))   # no dependence on the blocks' order
+    o = 0
+    for li, (ci, co, _) in enumerate(U.layers(s)):
+        for name, k in (("w", 9 * ci * co), ("b", co)):
+            a, b, c = g[o:o + k], g_o[o:o + k], g_64[o:o + k]
+            assert np.linalg.norm(a - c) <= 2.0 * np.linalg.norm(b - c) + 1e-6 * np.linalg.norm(c), (li, name)
+            o += k
+
+
 def test_training_reduces_loss(gpu_lib):
     """Fit a fixed linear map of the input (a smoothed combination of the
     channels) on one batch: 150 Adam steps cut the loss by 10x."""
