@@ -2,7 +2,7 @@
 //
 // A 2-D U-Net maps (m_x, m_y, m_z, film mask) on the plane of the MG box to
 // the box potential, one output channel per z plane of the box.  Weights and
-// activations are bf16 on the matrix cores (v_mfma_f32_16x16x16_bf16, FP32
+// activations are bf16 on the matrix cores (v_mfma_f32_16x16x32_bf16, FP32
 // accumulation); gradients, master weights and Adam moments are FP32.  All of
 // training runs here: forward, backward (data and weight gradients as
 // implicit GEMMs), loss and optimiser.  The multigrid solver still decides
@@ -43,10 +43,6 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kLevels = 4;
 constexpr int kNT = 256;
-// levels with at least this many pixels use 64-pixel waves (4 row tiles)
-constexpr int64_t kWideTileMinPixels = 65536;
-// dynamic LDS of a convolution block (the per-tap weight slice)
-constexpr size_t kConvLdsMax = 64 * 1024;
 
 __device__ __forceinline__ uint16_t f2bf(float f) {   // round to nearest even
     uint32_t u = __float_as_uint(f);
@@ -56,222 +52,304 @@ __device__ __forceinline__ uint16_t f2bf(float f) {   // round to nearest even
 __device__ __forceinline__ float bf2f(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
 
 
-// ---------------------------------------------------------------------------
-// 3x3 convolution as an implicit GEMM: rows = pixels, columns = output
-// channels, reduction = 9 taps x input channels.  A block is 4 waves; a wave
-// owns 16*MT pixels (MT 16-row MFMA tiles) x 16*NT channels; the 4 waves
-// share the block's channels.  Per tap, the block's weight slice
-// (16*NT rows of cin, rows padded by 8 elements against bank conflicts) is
-// staged in LDS once and read from there by all waves; the pixel operands are
-// 8-byte loads of 4 consecutive channels from global memory.  Also the data
-// gradient of a convolution: the same product of the output gradient with
-// the tap-flipped, transposed weights.
-// Requires: cin % 16 == 0, cout % (16*NT) == 0, xs, xo, ys, yo multiples of 4,
-// dynamic LDS of 16*NT*(cin+8)*2 bytes.
-// ---------------------------------------------------------------------------
-template <int MT, int NT, bool RELU, bool OUT_F32>
-__global__ __launch_bounds__(256) void k_conv3x3(const uint16_t *__restrict__ x, int xs, int xo, int cin,
-                                                 const uint16_t *__restrict__ w, const float *__restrict__ bias,
-                                                 void *__restrict__ y, int ys, int yo, int cout, int B, int H,
-                                                 int W) {
-    extern __shared__ __align__(16) unsigned char conv_smem[];
-    uint16_t *wsl = reinterpret_cast<uint16_t *>(conv_smem);
-    const int ws_row = cin + 8;   // LDS row stride of the weight slice (elements)
-    const int P = B * H * W;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int li = lane & 15, lk = (lane >> 4) * 4;
-    const int p_base = (blockIdx.x * 4 + wave) * (16 * MT);
-    const int co_base = blockIdx.y * (16 * NT);
-    int yl[MT], xl[MT];
-    bool pv[MT];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-        const int p = p_base + mt * 16 + li;
-        pv[mt] = p < P;
-        xl[mt] = p % W;
-        yl[mt] = (p / W) % H;
-    }
-    f32x4 acc[MT][NT];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int tap = 0; tap < 9; ++tap) {
-        const int dy = tap / 3 - 1, dx = tap % 3 - 1;
-        const uint16_t *xa[MT];
-        bool qv[MT];
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-            const int yy = yl[mt] + dy, xx = xl[mt] + dx;
-            qv[mt] = pv[mt] && yy >= 0 && yy < H && xx >= 0 && xx < W;
-            const int64_t q = (int64_t)(p_base + mt * 16 + li) + dy * W + dx;
-            xa[mt] = x + (qv[mt] ? q * xs + xo + lk : 0);
-        }
-        // stage w[tap][co_base .. co_base + 16 NT)[0 .. cin) (contiguous) in LDS, 16 bytes at a time
-        __syncthreads();   // the previous tap's reads are done
-        {
-            const uint4 *src = reinterpret_cast<const uint4 *>(w + ((int64_t)tap * cout + co_base) * cin);
-            const int per_row = cin / 8, total = 16 * NT * per_row;
-            for (int e = threadIdx.x; e < total; e += 256) {
-                const int row = e / per_row, c8 = e - row * per_row;
-                *reinterpret_cast<uint4 *>(wsl + row * ws_row + c8 * 8) = src[e];
-            }
-        }
-        __syncthreads();
-        const uint16_t *wt = wsl + li * ws_row + lk;
-        for (int ci0 = 0; ci0 < cin; ci0 += 16) {
-            bf16x4 a[MT], b[NT];
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
-                a[mt] = qv[mt] ? *(const bf16x4 *)(xa[mt] + ci0) : bf16x4{0, 0, 0, 0};
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) b[nt] = *(const bf16x4 *)(wt + nt * 16 * ws_row + ci0);
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-                for (int nt = 0; nt < NT; ++nt)
-                    acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[mt], b[nt], acc[mt][nt], 0, 0, 0);
-        }
-    }
-    // lane holds rows 4*(lane/16)+r, column lane%16 of every 16x16 tile
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-            const int co = co_base + nt * 16 + li;
-            const float bv = bias ? bias[co] : 0.f;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int p = p_base + mt * 16 + lk + r;
-                if (p >= P) continue;
-                float v = acc[mt][nt][r] + bv;
-                if (RELU) v = fmaxf(v, 0.f);
-                const int64_t o = (int64_t)p * ys + yo + co;
-                if (OUT_F32) ((float *)y)[o] = v;
-                else ((uint16_t *)y)[o] = f2bf(v);
-            }
-        }
+// Input of a convolution, channels last: channels [0, lo_c) are the nearest 2x
+// upsampling of a half-resolution tensor (dense lo_c channels, lo_c a multiple
+// of 32), the rest come from a dense tensor of hi_c channels at the output's
+// resolution.  So a decoder's concatenation [up, skip] is never stored.
+struct ConvSrc {
+    const uint16_t *lo;
+    int lo_c;
+    const uint16_t *hi;
+    int hi_c;
+};
+// The value, hidden from the optimiser: addresses formed from it are recomputed
+// where they are used instead of being kept in registers over a block's loops.
+__device__ __forceinline__ int opaque(int v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+// the 8 channels from c on of pixel (b, yy, xx), zero outside the image
+__device__ __forceinline__ uint4 src_load(const ConvSrc &s, int c, bool low, int b, int yy, int xx, int H, int W) {
+    if (yy < 0 || yy >= H || xx < 0 || xx >= W) return uint4{0u, 0u, 0u, 0u};
+    const uint16_t *p = low ? s.lo + ((int64_t)(b * (H >> 1) + (yy >> 1)) * (W >> 1) + (xx >> 1)) * s.lo_c + c
+                            : s.hi + ((int64_t)(b * H + yy) * W + xx) * s.hi_c + (c - s.lo_c);
+    return *reinterpret_cast<const uint4 *>(p);
 }
 
-// 3x3 convolution on spatial tiles (gfx950's K = 32 bf16 matrix-core
-// product, v_mfma_f32_16x16x32_bf16): a block computes a TH x 32 pixel tile
-// of one image for 16*NT output channels.  Input channels go in chunks of
-// 32: the chunk's input tile with its one-pixel halo ((TH+2) x 34 pixels,
-// zero outside the image) and the chunk's weights of all nine taps are staged
-// in LDS once, then every tap's product reads both from LDS, so each input
-// pixel is read from memory once per chunk instead of once per tap.  Wave w
-// owns rows w*TH/4 .. of the tile (16-pixel half rows as MFMA row tiles) and
-// all 16*NT channels.  The same product as k_conv3x3 (also used for the data
-// gradient); it needs the pixel slices 16-byte aligned (xs, xo multiples of
-// 8).  LDS rows are padded by 8 elements against bank conflicts.
-constexpr int kTileW = 32, kTileKC = 32, kTileRow = kTileKC + 8;
-template <int TH, int NT>
-constexpr size_t conv_tile_lds() {
-    return sizeof(uint16_t) * (size_t)kTileRow * ((TH + 2) * (kTileW + 2) + 9 * 16 * NT);
+// What a convolution does with its sums (in FP32 registers):
+//  ACT   bf16 of relu(sum + bias) to y; with pool also its 2x2 average
+//  F32   sum (+ bias) to yf
+//  MASK  bf16 of the sum where mask > 0, else 0, to y: a data gradient and the
+//        ReLU backward of the layer before it
+//  MSE   the loss's terms of sum + bias against tgt (channels < cv, pixels
+//        x < wv, y < hv) added to *loss, and the bf16 of the loss gradient to y
+//  CAT   data gradient of a concatenation [up, skip]: channels < up_c are summed
+//        over 2x2 pixels (the upsampling's gradient) and masked into y at half
+//        resolution, the rest go to yf in FP32
+enum { EPI_ACT, EPI_F32, EPI_MASK, EPI_MSE, EPI_CAT };
+struct ConvEpi {
+    uint16_t *y = nullptr;
+    float *yf = nullptr;
+    uint16_t *pool = nullptr;
+    const uint16_t *mask = nullptr;
+    int up_c = 0;
+    const uint16_t *tgt = nullptr;
+    int cv = 0, wv = 0, hv = 0;
+    double inv_count = 0.0;
+    double *loss = nullptr;
+};
+
+__device__ __forceinline__ uint4 relu_mask(uint4 v, uint4 m) {
+    uint16_t *hv = reinterpret_cast<uint16_t *>(&v);
+    const uint16_t *hm = reinterpret_cast<const uint16_t *>(&m);
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+        if (!(bf2f(hm[k]) > 0.f)) hv[k] = 0;
+    return v;
 }
-template <int TH, int NT, bool RELU, bool OUT_F32>
-__global__ __launch_bounds__(256) void k_conv3x3_tile(const uint16_t *__restrict__ x, int xs, int xo, int cin,
-                                                      const uint16_t *__restrict__ w, const float *__restrict__ bias,
-                                                      void *__restrict__ y, int ys, int yo, int cout, int B, int H,
-                                                      int W) {
-    constexpr int RW = TH / 4;           // tile rows per wave
-    constexpr int MT = 2 * RW;           // 16-pixel row tiles per wave
-    constexpr int CO = 16 * NT;          // output channels of the block
-    constexpr int TPW = kTileW + 2;      // tile width with halo
-    constexpr int NIN = (TH + 2) * TPW;  // staged input pixels
-    extern __shared__ __align__(16) unsigned char tile_smem[];
-    uint16_t *xin = reinterpret_cast<uint16_t *>(tile_smem);   // [NIN][kTileRow]
-    uint16_t *wsl = xin + NIN * kTileRow;                      // [9][CO][kTileRow]
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int li = lane & 15, kg = (lane >> 4) * 8;
-    const int ntx = (W + kTileW - 1) / kTileW, nty = (H + TH - 1) / TH;
-    const int tx = blockIdx.x % ntx, ty = (blockIdx.x / ntx) % nty, b = blockIdx.x / (ntx * nty);
-    const int x0 = tx * kTileW, y0 = ty * TH;
-    const int co_base = blockIdx.y * CO;
-    f32x4 acc[MT][NT];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    // A chunk's input tile and weights go through registers: the next chunk's
-    // loads are issued before the current chunk's products, so they are in
-    // flight while the matrix cores work.
-    constexpr int NI = (NIN * (kTileKC / 8) + 255) / 256, NW = (9 * CO * (kTileKC / 8) + 255) / 256;
+
+// 3x3 convolution as an implicit GEMM on gfx950's K = 32 bf16 matrix-core
+// product: rows = pixels, columns = output channels, reduction = 9 taps x input
+// channels.  Also the data gradient (the output gradient with tap-flipped,
+// transposed weights).  A block computes TH x 16*TW pixels for 16*NT output
+// channels; wave w owns TH/4 pixel rows.  Input channels go in chunks of 32: a
+// chunk's haloed input tile and its weights of all nine taps are staged in LDS
+// through registers, the next chunk's loads in flight during the products.
+//
+// LDS reads bound a straightforward loop over taps (one input operand per
+// product pair), so the nine taps' weights are held in registers and the
+// wave walks the input rows once: input row i serves output rows i, i-1, i-2
+// (taps dy = 0, 1, 2), a third of the reads.  Per chunk and wave of the 16 x 32
+// tile: 54 KB of LDS reads for 144 products, 93 of the CU's 128 bytes per clock
+// at the matrix cores' full rate.  Every sum still takes its chunks in order and
+// within a chunk its taps 0..8.
+//
+// The sums leave through LDS as whole 16-byte pieces of a pixel (two-byte stores
+// of the product's own layout took as long as the products), with the pass that
+// would follow (pooling, upsampling, the ReLU's gradient, the loss) applied on
+// the way out.  A layer of one chunk keeps its weights in LDS over a block's run
+// of tiles.
+// Requires cin % 16 == 0, cout % (16*NT) == 0; H, W even for pool and CAT.
+// Measured against the tap-by-tap tile kernel with separate pooling, upsampling,
+// concatenation, ReLU-gradient and loss passes: forward at 528 x 528 467 -> 365
+// us, training step at batch 8 8.10 -> 5.84 ms.
+constexpr int kKC = 32, kKRow = kKC + 8;   // channel chunk; LDS row, padded against bank conflicts
+template <int TH, int TW, int NT>
+struct ConvShape {
+    static constexpr int CO = 16 * NT, XW = 16 * TW + 2, NPX = (TH + 2) * XW, NOUT = TH * 16 * TW;
+    static constexpr int kXin = NPX * kKRow, kOut = NOUT * (CO + 8), kReg = kXin > kOut ? kXin : kOut;
+    static constexpr size_t LDS = sizeof(uint16_t) * (size_t)(kReg + 9 * CO * kKRow);
+};
+template <int TH, int TW, int NT, int EPI, bool RELU>
+__global__ __launch_bounds__(256, 2) void k_conv3x3(ConvSrc src, int cin, const uint16_t *__restrict__ w,
+                                                    const float *__restrict__ bias, ConvEpi ep, int cout, int B,
+                                                    int H, int W) {
+    using S = ConvShape<TH, TW, NT>;
+    constexpr int RW = TH / 4, CO = S::CO, XW = S::XW, NPX = S::NPX, OROW = CO + 8;
+    extern __shared__ __align__(16) unsigned char conv_smem[];
+    uint16_t *xin = reinterpret_cast<uint16_t *>(conv_smem);   // [NPX][kKRow], later the output tile [pixel][OROW]
+    uint16_t *wl = xin + S::kReg;                              // [9][CO][kKRow]
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 15, g = lane >> 4;
+    const int ntx = (W + 16 * TW - 1) / (16 * TW), nty = (H + TH - 1) / TH, ntile = ntx * nty * B;
+    const int t0 = (int)((int64_t)ntile * blockIdx.x / gridDim.x),
+              t1 = (int)((int64_t)ntile * (blockIdx.x + 1) / gridDim.x);
+    const int co_base = (int)blockIdx.y * CO;
+    const bool one_chunk = cin <= kKC;
+    constexpr int NI = (NPX * 4 + 255) / 256, NW = (9 * CO * 4 + 255) / 256;
     uint4 ri[NI], rw[NW];
-    auto fetch = [&](int c0) {
+    auto fetch_x = [&](int t, int c0) {
+        const int x0 = (t % ntx) * 16 * TW, y0 = ((t / ntx) % nty) * TH, b = t / (ntx * nty);
+        const bool low = c0 < src.lo_c;
+        const int tid = opaque(threadIdx.x);
 #pragma unroll
         for (int k = 0; k < NI; ++k) {
-            const int e = threadIdx.x + k * 256;
-            const int pix = e >> 2, c = c0 + (e & 3) * 8;
-            const int yy = y0 + pix / TPW - 1, xx = x0 + pix % TPW - 1;
+            const int e = tid + k * 256, pix = e >> 2, c = c0 + (e & 3) * 8;
             ri[k] = uint4{0u, 0u, 0u, 0u};
-            if (e < NIN * 4 && yy >= 0 && yy < H && xx >= 0 && xx < W && c < cin)
-                ri[k] = *reinterpret_cast<const uint4 *>(x + ((int64_t)(b * H + yy) * W + xx) * xs + xo + c);
+            if (e < NPX * 4 && c < cin) ri[k] = src_load(src, c, low, b, y0 + pix / XW - 1, x0 + pix % XW - 1, H, W);
         }
+    };
+    auto fetch_w = [&](int c0) {
+        const int tid = opaque(threadIdx.x);
 #pragma unroll
         for (int k = 0; k < NW; ++k) {
-            const int e = threadIdx.x + k * 256;
-            const int row = e >> 2, c = c0 + (e & 3) * 8;   // row = tap * CO + co
+            const int e = tid + k * 256, row = e >> 2, c = c0 + (e & 3) * 8;   // row = tap * CO + co
             const int tap = row / CO, co = row - tap * CO;
             rw[k] = uint4{0u, 0u, 0u, 0u};
             if (e < 9 * CO * 4 && c < cin)
                 rw[k] = *reinterpret_cast<const uint4 *>(w + ((int64_t)tap * cout + co_base + co) * cin + c);
         }
     };
-    fetch(0);
-    for (int c0 = 0; c0 < cin; c0 += kTileKC) {
-        __syncthreads();   // the previous chunk's reads are done
+    double lsum = 0.0;
+    if (t0 < t1) {
+        fetch_x(t0, 0);
+        fetch_w(0);
+    }
+    for (int t = t0; t < t1; ++t) {
+        const int x0 = (t % ntx) * 16 * TW, y0 = ((t / ntx) % nty) * TH, b = t / (ntx * nty);
+        f32x4 acc[RW][TW][NT];
 #pragma unroll
-        for (int k = 0; k < NI; ++k) {
-            const int e = threadIdx.x + k * 256;
-            if (e < NIN * 4) *reinterpret_cast<uint4 *>(xin + (e >> 2) * kTileRow + (e & 3) * 8) = ri[k];
-        }
+        for (int r = 0; r < RW; ++r)
 #pragma unroll
-        for (int k = 0; k < NW; ++k) {
-            const int e = threadIdx.x + k * 256;
-            if (e < 9 * CO * 4) *reinterpret_cast<uint4 *>(wsl + (e >> 2) * kTileRow + (e & 3) * 8) = rw[k];
-        }
-        __syncthreads();
-        if (c0 + kTileKC < cin) fetch(c0 + kTileKC);
+            for (int h = 0; h < TW; ++h)
 #pragma unroll
-        for (int tap = 0; tap < 9; ++tap) {
-            const int dy = tap / 3, dx = tap % 3;   // offsets into the haloed tile
-            bf16x8 a[MT], bw[NT];
+                for (int nt = 0; nt < NT; ++nt) acc[r][h][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int c0 = 0; c0 < cin; c0 += kKC) {
+            __syncthreads();   // the previous chunk's (or output tile's) reads are done
 #pragma unroll
-            for (int mt = 0; mt < MT; ++mt) {
-                const int r = wave * RW + (mt >> 1), col = (mt & 1) * 16 + li;
-                a[mt] = *reinterpret_cast<const bf16x8 *>(xin + ((r + dy) * TPW + col + dx) * kTileRow + kg);
+            for (int k = 0; k < NI; ++k) {
+                const int e = threadIdx.x + k * 256;
+                if (e < NPX * 4) *reinterpret_cast<uint4 *>(xin + (e >> 2) * kKRow + (e & 3) * 8) = ri[k];
             }
+            if (!one_chunk || t == t0) {
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt)
-                bw[nt] = *reinterpret_cast<const bf16x8 *>(wsl + (tap * CO + nt * 16 + li) * kTileRow + kg);
+                for (int k = 0; k < NW; ++k) {
+                    const int e = threadIdx.x + k * 256;
+                    if (e < 9 * CO * 4) *reinterpret_cast<uint4 *>(wl + (e >> 2) * kKRow + (e & 3) * 8) = rw[k];
+                }
+            }
+            __syncthreads();
+            if (c0 + kKC < cin) {
+                fetch_x(t, c0 + kKC);
+                fetch_w(c0 + kKC);
+            } else if (t + 1 < t1) {
+                fetch_x(t + 1, 0);
+                if (!one_chunk) fetch_w(0);
+            }
+            bf16x8 bw[9][NT];
 #pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
+            for (int tap = 0; tap < 9; ++tap)
 #pragma unroll
                 for (int nt = 0; nt < NT; ++nt)
-                    acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[mt], bw[nt], acc[mt][nt], 0, 0, 0);
-        }
-    }
-    // lane holds pixels 4*(lane/16)+r of each 16-pixel row tile, channel lane%16
+                    bw[tap][nt] = *reinterpret_cast<const bf16x8 *>(wl + (tap * CO + nt * 16 + li) * kKRow + g * 8);
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-        const int yy = y0 + wave * RW + (mt >> 1);
-        if (yy >= H) continue;
+            for (int i = 0; i < RW + 2; ++i) {
+                bf16x8 a[3][TW];
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-            const int co = co_base + nt * 16 + li;
-            const float bv = bias ? bias[co] : 0.f;
+                for (int dx = 0; dx < 3; ++dx)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int xx = x0 + (mt & 1) * 16 + (lane >> 4) * 4 + r;
-                if (xx >= W) continue;
-                float v = acc[mt][nt][r] + bv;
-                if (RELU) v = fmaxf(v, 0.f);
-                const int64_t o = ((int64_t)(b * H + yy) * W + xx) * ys + yo + co;
-                if (OUT_F32) ((float *)y)[o] = v;
-                else ((uint16_t *)y)[o] = f2bf(v);
+                    for (int h = 0; h < TW; ++h)
+                        a[dx][h] = *reinterpret_cast<const bf16x8 *>(
+                            xin + ((wave * RW + i) * XW + h * 16 + li + dx) * kKRow + g * 8);
+#pragma unroll
+                for (int dy = 0; dy < 3; ++dy) {
+                    const int r = i - dy;
+                    if (r < 0 || r >= RW) continue;
+#pragma unroll
+                    for (int dx = 0; dx < 3; ++dx)
+#pragma unroll
+                        for (int h = 0; h < TW; ++h)
+#pragma unroll
+                            for (int nt = 0; nt < NT; ++nt)
+                                acc[r][h][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                                    a[dx][h], bw[dy * 3 + dx][nt], acc[r][h][nt], 0, 0, 0);
+                }
             }
         }
+        // lane holds pixels 4 g + q of each 16-pixel tile, channel li
+        const bool cat_up = EPI == EPI_CAT && co_base < ep.up_c;
+        if (EPI == EPI_F32 || (EPI == EPI_CAT && !cat_up)) {
+            const int cs = EPI == EPI_CAT ? cout - ep.up_c : cout, cb = EPI == EPI_CAT ? co_base - ep.up_c : co_base;
+#pragma unroll
+            for (int r = 0; r < RW; ++r) {
+                const int yy = y0 + wave * RW + r;
+                if (yy >= H) continue;
+#pragma unroll
+                for (int h = 0; h < TW; ++h)
+#pragma unroll
+                    for (int nt = 0; nt < NT; ++nt) {
+                        const int co = nt * 16 + li;
+                        const float bv = bias ? bias[co_base + co] : 0.f;
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            const int xx = x0 + h * 16 + g * 4 + q;
+                            if (xx < W) ep.yf[((int64_t)(b * H + yy) * W + xx) * cs + cb + co] = acc[r][h][nt][q] + bv;
+                        }
+                    }
+            }
+            continue;
+        }
+        __syncthreads();   // every wave's reads of xin are done
+        if (cat_up) {
+            if constexpr (EPI == EPI_CAT) {
+#pragma unroll
+                for (int r = 0; r < RW; r += 2)
+#pragma unroll
+                    for (int h = 0; h < TW; ++h)
+#pragma unroll
+                        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                            for (int q = 0; q < 4; q += 2) {
+                                const float v = acc[r][h][nt][q] + acc[r][h][nt][q + 1] + acc[r + 1][h][nt][q] +
+                                                acc[r + 1][h][nt][q + 1];
+                                const int px = ((wave * RW + r) / 2) * 8 * TW + h * 8 + (g * 4 + q) / 2;
+                                xin[px * OROW + nt * 16 + li] = f2bf(v);
+                            }
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < RW; ++r)
+#pragma unroll
+                for (int h = 0; h < TW; ++h)
+#pragma unroll
+                    for (int nt = 0; nt < NT; ++nt) {
+                        const int co = co_base + nt * 16 + li;
+                        const float bv = bias ? bias[co] : 0.f;
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            float v = acc[r][h][nt][q] + bv;
+                            if (RELU) v = fmaxf(v, 0.f);
+                            if constexpr (EPI == EPI_MSE) {
+                                const int yy = y0 + wave * RW + r, xx = x0 + h * 16 + g * 4 + q;
+                                float gr = 0.f;
+                                if (co < ep.cv && xx < ep.wv && yy < ep.hv) {
+                                    const double d =
+                                        (double)v - (double)bf2f(ep.tgt[((int64_t)(b * H + yy) * W + xx) * cout + co]);
+                                    lsum += d * d;
+                                    gr = (float)(2.0 * d * ep.inv_count);
+                                }
+                                v = gr;
+                            }
+                            xin[((wave * RW + r) * 16 * TW + h * 16 + g * 4 + q) * OROW + nt * 16 + li] = f2bf(v);
+                        }
+                    }
+        }
+        __syncthreads();
+        // out of LDS in 16-byte pieces (8 channels of a pixel)
+        const int tid = opaque(threadIdx.x);
+        const int sh = cat_up ? 1 : 0;   // CAT: half resolution
+        const int Ho = H >> sh, Wo = W >> sh, co_n = cat_up ? ep.up_c : cout, ow = (16 * TW) >> sh;
+        constexpr int P8 = CO / 8;
+        for (int e = tid; e < ((TH * 16 * TW) >> (2 * sh)) * P8; e += 256) {
+            const int px = e / P8, c = (e % P8) * 8;
+            const int yy = (y0 >> sh) + px / ow, xx = (x0 >> sh) + px % ow;
+            if (yy >= Ho || xx >= Wo) continue;
+            uint4 v = *reinterpret_cast<const uint4 *>(xin + px * OROW + c);
+            const int64_t o = ((int64_t)(b * Ho + yy) * Wo + xx) * co_n + co_base + c;
+            if (EPI == EPI_MASK || EPI == EPI_CAT) v = relu_mask(v, *reinterpret_cast<const uint4 *>(ep.mask + o));
+            *reinterpret_cast<uint4 *>(ep.y + o) = v;
+        }
+        if (EPI == EPI_ACT && ep.pool) {
+            for (int e = tid; e < (TH / 2 * 8 * TW) * P8; e += 256) {
+                const int px = e / P8, c = (e % P8) * 8, py = px / (8 * TW), pxx = px % (8 * TW);
+                const int yy = (y0 >> 1) + py, xx = (x0 >> 1) + pxx;
+                if (yy >= (H >> 1) || xx >= (W >> 1)) continue;
+                const uint16_t *q0 = xin + (2 * py * 16 * TW + 2 * pxx) * OROW + c;
+                const uint16_t *q1 = q0 + OROW, *q2 = q0 + 16 * TW * OROW, *q3 = q2 + OROW;
+                uint4 o;
+                uint16_t *ho = reinterpret_cast<uint16_t *>(&o);
+#pragma unroll
+                for (int k = 0; k < 8; ++k)
+                    ho[k] = f2bf(0.25f * (bf2f(q0[k]) + bf2f(q1[k]) + bf2f(q2[k]) + bf2f(q3[k])));
+                *reinterpret_cast<uint4 *>(ep.pool + ((int64_t)(b * (H >> 1) + yy) * (W >> 1) + xx) * cout + co_base + c) = o;
+            }
+        }
+    }
+    if constexpr (EPI == EPI_MSE) {
+        __shared__ double lpart[4];
+        for (int o = 32; o > 0; o >>= 1) lsum += __shfl_xor(lsum, o);
+        if (lane == 0) lpart[wave] = lsum;
+        __syncthreads();
+        if (threadIdx.x == 0) atomicAdd(ep.loss, (lpart[0] + lpart[1] + lpart[2] + lpart[3]) * ep.inv_count);
     }
 }
 
@@ -296,9 +374,8 @@ __global__ __launch_bounds__(256) void k_conv3x3_tile(const uint16_t *__restrict
 // 8 x 528 x 528 step (742 -> 84 us per 32 x 32 tiled layer).
 constexpr int kWgT = 16, kWgX = kWgT + 2;   // pixel tile and tile with halo
 template <int MT, int NT>
-__global__ __launch_bounds__(256, 2) void k_conv3x3_wgrad(const uint16_t *__restrict__ dz, int cout,
-                                                          const uint16_t *__restrict__ x, int xs, int xo, int cin,
-                                                          float *__restrict__ part, int B, int H, int W) {
+__global__ __launch_bounds__(256, 2) void k_conv3x3_wgrad(const uint16_t *__restrict__ dz, int cout, ConvSrc src,
+                                                          int cin, float *__restrict__ part, int B, int H, int W) {
     constexpr int CO = 16 * MT, CI = 16 * NT;
     constexpr int NX = kWgX * kWgX * (CI / 8), NZ = kWgT * kWgT * (CO / 8);   // 16-byte pieces of a tile
     constexpr int LX = (NX + 255) / 256, LZ = (NZ + 255) / 256;
@@ -321,6 +398,7 @@ __global__ __launch_bounds__(256, 2) void k_conv3x3_wgrad(const uint16_t *__rest
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) acc[tap][mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
+    const bool low = ci_base < src.lo_c;
     uint4 rx[LX], rz[LZ];
     auto fetch = [&](int t) {
         const int tx = t % ntx, ty = (t / ntx) % nty, b = t / (ntx * nty);
@@ -328,10 +406,9 @@ __global__ __launch_bounds__(256, 2) void k_conv3x3_wgrad(const uint16_t *__rest
 #pragma unroll
         for (int k = 0; k < LX; ++k) {
             const int e = threadIdx.x + k * 256, pix = e / (CI / 8), c = (e % (CI / 8)) * 8;
-            const int yy = y0 + pix / kWgX - 1, xx = x0 + pix % kWgX - 1;
             rx[k] = uint4{0u, 0u, 0u, 0u};
-            if (e < NX && yy >= 0 && yy < H && xx >= 0 && xx < W)
-                rx[k] = *reinterpret_cast<const uint4 *>(x + ((int64_t)(b * H + yy) * W + xx) * xs + xo + ci_base + c);
+            if (e < NX)
+                rx[k] = src_load(src, ci_base + c, low, b, y0 + pix / kWgX - 1, x0 + pix % kWgX - 1, H, W);
         }
 #pragma unroll
         for (int k = 0; k < LZ; ++k) {
@@ -446,173 +523,32 @@ __global__ __launch_bounds__(256) void k_part_sum(const float *__restrict__ part
     if (g == 0 && i < n) out[i] = (red[0][c] + red[1][c]) + (red[2][c] + red[3][c]);
 }
 
-// 2x2 average pool of a slice: y[b][Y][X][c] = mean of x[b][2Y+i][2X+j][xo+c]
-__global__ void k_pool2(const uint16_t *__restrict__ x, int xs, int xo, int C, uint16_t *__restrict__ y, int B,
-                        int H, int W) {
-    const int Hc = H / 2, Wc = W / 2;
-    const int64_t n = (int64_t)B * Hc * Wc * C;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const int c = (int)(i % C);
-        const int64_t pc = i / C;
-        const int X = (int)(pc % Wc), Y = (int)((pc / Wc) % Hc), b = (int)(pc / ((int64_t)Wc * Hc));
-        const int64_t p00 = ((int64_t)b * H + 2 * Y) * W + 2 * X;
-        float s = bf2f(x[p00 * xs + xo + c]) + bf2f(x[(p00 + 1) * xs + xo + c]) + bf2f(x[(p00 + W) * xs + xo + c]) +
-                  bf2f(x[(p00 + W + 1) * xs + xo + c]);
-        y[i] = f2bf(0.25f * s);
-    }
-}
-
-// k_pool2 eight channels (16 bytes) at a time: C, xs, xo multiples of 8
-__global__ void k_pool2_v8(const uint16_t *__restrict__ x, int xs, int xo, int C, uint16_t *__restrict__ y, int B,
-                           int H, int W) {
-    const int Hc = H / 2, Wc = W / 2, C8 = C / 8;
-    const int64_t n = (int64_t)B * Hc * Wc * C8;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const int c = (int)(i % C8) * 8;
-        const int64_t pc = i / C8;
-        const int X = (int)(pc % Wc), Y = (int)((pc / Wc) % Hc), b = (int)(pc / ((int64_t)Wc * Hc));
-        const int64_t p00 = ((int64_t)b * H + 2 * Y) * W + 2 * X;
-        const uint4 q[4] = {*reinterpret_cast<const uint4 *>(x + p00 * xs + xo + c),
-                            *reinterpret_cast<const uint4 *>(x + (p00 + 1) * xs + xo + c),
-                            *reinterpret_cast<const uint4 *>(x + (p00 + W) * xs + xo + c),
-                            *reinterpret_cast<const uint4 *>(x + (p00 + W + 1) * xs + xo + c)};
-        const uint16_t *h[4] = {reinterpret_cast<const uint16_t *>(&q[0]), reinterpret_cast<const uint16_t *>(&q[1]),
-                                reinterpret_cast<const uint16_t *>(&q[2]), reinterpret_cast<const uint16_t *>(&q[3])};
-        uint4 o;
-        uint16_t *ho = reinterpret_cast<uint16_t *>(&o);
-#pragma unroll
-        for (int k = 0; k < 8; ++k) ho[k] = f2bf(0.25f * (bf2f(h[0][k]) + bf2f(h[1][k]) + bf2f(h[2][k]) + bf2f(h[3][k])));
-        *reinterpret_cast<uint4 *>(y + pc * C + c) = o;
-    }
-}
-
-// gradient of k_pool2: dx[fine][c] += 0.25 dy[coarse][c]   (dense C, FP32)
-__global__ void k_pool2_bwd(const float *__restrict__ dy, int C, float *__restrict__ dx, int B, int H, int W) {
-    const int64_t n = (int64_t)B * H * W * C;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const int c = (int)(i % C);
-        const int64_t p = i / C;
-        const int x = (int)(p % W), yy = (int)((p / W) % H), b = (int)(p / ((int64_t)W * H));
-        const int64_t pc = ((int64_t)b * (H / 2) + yy / 2) * (W / 2) + x / 2;
-        dx[i] += 0.25f * dy[pc * C + c];
-    }
-}
-
-// nearest 2x upsample into a slice: y[fine][yo+c] = x[coarse][c] (x dense C)
-__global__ void k_up2(const uint16_t *__restrict__ x, int C, uint16_t *__restrict__ y, int ys, int yo, int B, int H,
-                      int W) {
-    const int64_t n = (int64_t)B * H * W * C;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const int c = (int)(i % C);
-        const int64_t p = i / C;
-        const int xx = (int)(p % W), yy = (int)((p / W) % H), b = (int)(p / ((int64_t)W * H));
-        const int64_t pc = ((int64_t)b * (H / 2) + yy / 2) * (W / 2) + xx / 2;
-        y[p * ys + yo + c] = x[pc * C + c];
-    }
-}
-
-// k_up2 eight channels (16 bytes) at a time: C, ys, yo multiples of 8
-__global__ void k_up2_v8(const uint16_t *__restrict__ x, int C, uint16_t *__restrict__ y, int ys, int yo, int B,
-                         int H, int W) {
+// Gradient of an encoder's output, eight channels per thread: its skip part
+// plus a quarter of the pooled tensor's gradient, masked by the ReLU, as bf16:
+// dz[fine][c] = bf16((gs[fine][c] + 0.25 gp[coarse][c]) where y > 0)
+__global__ void k_skip_pool_relu(const float *__restrict__ gs, const float *__restrict__ gp,
+                                 const uint16_t *__restrict__ y, int C, uint16_t *__restrict__ dz, int B, int H,
+                                 int W) {
     const int C8 = C / 8;
     const int64_t n = (int64_t)B * H * W * C8;
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
         const int c = (int)(i % C8) * 8;
         const int64_t p = i / C8;
-        const int xx = (int)(p % W), yy = (int)((p / W) % H), b = (int)(p / ((int64_t)W * H));
-        const int64_t pc = ((int64_t)b * (H / 2) + yy / 2) * (W / 2) + xx / 2;
-        *reinterpret_cast<uint4 *>(y + p * ys + yo + c) = *reinterpret_cast<const uint4 *>(x + pc * C + c);
-    }
-}
-
-// gradient of k_up2: dx[coarse][c] = sum of the four dy[fine][yo+c]
-__global__ void k_up2_bwd(const float *__restrict__ dy, int ys, int yo, int C, float *__restrict__ dx, int B, int H,
-                          int W) {
-    const int Hc = H / 2, Wc = W / 2;
-    const int64_t n = (int64_t)B * Hc * Wc * C;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const int c = (int)(i % C);
-        const int64_t pc = i / C;
-        const int X = (int)(pc % Wc), Y = (int)((pc / Wc) % Hc), b = (int)(pc / ((int64_t)Wc * Hc));
-        const int64_t p00 = ((int64_t)b * H + 2 * Y) * W + 2 * X;
-        dx[i] = dy[p00 * ys + yo + c] + dy[(p00 + 1) * ys + yo + c] + dy[(p00 + W) * ys + yo + c] +
-                dy[(p00 + W + 1) * ys + yo + c];
-    }
-}
-
-// dst[p][c] = src[p][so+c]  (the skip part of a concatenation's gradient)
-__global__ void k_slice_copy(const float *__restrict__ src, int ss, int so, int C, float *__restrict__ dst, int64_t P) {
-    const int64_t n = P * C;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const int c = (int)(i % C);
-        dst[i] = src[(i / C) * ss + so + c];
-    }
-}
-
-// dz = bf16(dy * [y > 0]) with y a slice (ReLU layers), or bf16(dy) (y null)
-// k_relu_bwd eight channels per thread: C, ys, yo multiples of 8
-__global__ void k_relu_bwd_v8(const float *__restrict__ dy, const uint16_t *__restrict__ y, int ys, int yo, int C,
-                              uint16_t *__restrict__ dz, int64_t P) {
-    const int C8 = C / 8;
-    const int64_t n = P * C8;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t p = i / C8;
-        const int c = (int)(i - p * C8) * 8;
-        const float4 g0 = *reinterpret_cast<const float4 *>(dy + p * C + c);
-        const float4 g1 = *reinterpret_cast<const float4 *>(dy + p * C + c + 4);
-        float g[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
-        if (y) {
-            const uint4 q = *reinterpret_cast<const uint4 *>(y + p * ys + yo + c);
-            const uint16_t *h = reinterpret_cast<const uint16_t *>(&q);
-#pragma unroll
-            for (int k = 0; k < 8; ++k)
-                if (!(bf2f(h[k]) > 0.f)) g[k] = 0.f;
-        }
+        const int x = (int)(p % W), yy = (int)((p / W) % H), b = (int)(p / ((int64_t)W * H));
+        const int64_t pc = ((int64_t)b * (H / 2) + yy / 2) * (W / 2) + x / 2;
+        const float4 s0 = *reinterpret_cast<const float4 *>(gs + p * C + c),
+                     s1 = *reinterpret_cast<const float4 *>(gs + p * C + c + 4),
+                     q0 = *reinterpret_cast<const float4 *>(gp + pc * C + c),
+                     q1 = *reinterpret_cast<const float4 *>(gp + pc * C + c + 4);
+        const float v[8] = {s0.x + 0.25f * q0.x, s0.y + 0.25f * q0.y, s0.z + 0.25f * q0.z, s0.w + 0.25f * q0.w,
+                            s1.x + 0.25f * q1.x, s1.y + 0.25f * q1.y, s1.z + 0.25f * q1.z, s1.w + 0.25f * q1.w};
         uint4 o;
         uint16_t *ho = reinterpret_cast<uint16_t *>(&o);
 #pragma unroll
-        for (int k = 0; k < 8; ++k) ho[k] = f2bf(g[k]);
-        *reinterpret_cast<uint4 *>(dz + p * C + c) = o;
+        for (int k = 0; k < 8; ++k) ho[k] = f2bf(v[k]);
+        *reinterpret_cast<uint4 *>(dz + p * C + c) =
+            relu_mask(o, *reinterpret_cast<const uint4 *>(y + p * C + c));
     }
-}
-
-__global__ void k_relu_bwd(const float *__restrict__ dy, const uint16_t *__restrict__ y, int ys, int yo, int C,
-                           uint16_t *__restrict__ dz, int64_t P) {
-    const int64_t n = P * C;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        float g = dy[i];
-        if (y) {
-            const int c = (int)(i % C);
-            if (!(bf2f(y[(i / C) * ys + yo + c]) > 0.f)) g = 0.f;
-        }
-        dz[i] = f2bf(g);
-    }
-}
-
-// Mean squared error over channels < cv and pixels with x < wv, y < hv:
-// loss += sum diff^2 (FP64 atomics per block), dpred = 2 diff * inv_count.
-__global__ __launch_bounds__(256) void k_mse(const float *__restrict__ pred, const uint16_t *__restrict__ tgt, int C,
-                                             int cv, int wv, int hv, int B, int H, int W, double inv_count,
-                                             float *__restrict__ dpred, double *__restrict__ loss) {
-    __shared__ double part[4];
-    const int64_t n = (int64_t)B * H * W * C;
-    double s = 0.0;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const int c = (int)(i % C);
-        const int64_t p = i / C;
-        const int x = (int)(p % W), y = (int)((p / W) % H);
-        float g = 0.f;
-        if (c < cv && x < wv && y < hv) {
-            const double d = (double)pred[i] - (double)bf2f(tgt[i]);
-            s += d * d;
-            g = (float)(2.0 * d * inv_count);
-        }
-        dpred[i] = g;
-    }
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) atomicAdd(loss, (part[0] + part[1] + part[2] + part[3]) * inv_count);
 }
 
 // Adam (Kingma & Ba 2015) on FP32 master parameters; bc1 = 1 - b1^t, bc2 = 1 - b2^t
@@ -717,13 +653,14 @@ struct UNet {
     int64_t t = 0;                // Adam step count
     double *d_loss = nullptr, *h_loss = nullptr;
     std::vector<void *> bufs;
-    // activations (bf16): per level
-    uint16_t *ea[kLevels] = {}, *eb[kLevels] = {}, *pool[kLevels] = {}, *cat[kLevels] = {}, *da[kLevels] = {},
-             *db[kLevels] = {}, *dz[kLevels] = {};
-    float *out = nullptr;
-    // gradients (FP32)
-    float *g_out = nullptr, *g_a[kLevels] = {}, *g_b[kLevels] = {}, *g_cat[kLevels] = {}, *g_eb[kLevels] = {},
-          *g_pool[kLevels] = {};
+    // activations (bf16), dense, per level: encoder outputs of the two
+    // convolutions, pooled input, decoder outputs
+    uint16_t *ea[kLevels] = {}, *eb[kLevels] = {}, *pool[kLevels] = {}, *da[kLevels] = {}, *db[kLevels] = {};
+    // output gradients (bf16): a layer reads one and writes the other
+    uint16_t *dz[kLevels][2] = {};
+    // gradients that meet another before they are rounded (FP32): skip
+    // connections and pooled inputs
+    float *g_skip[kLevels] = {}, *g_pool[kLevels] = {};
 
     int c(int l) const { return base << l; }
     int hl(int l) const { return H >> l; }
@@ -789,26 +726,18 @@ struct UNet {
             for (int l = 0; l < kLevels; ++l) {
                 const int64_t P = pl(l);
                 ea[l] = dalloc<uint16_t>(P * c(l));
-                if (l == kLevels - 1) eb[l] = dalloc<uint16_t>(P * c(l));
-                else {
-                    cat[l] = dalloc<uint16_t>(P * (c(l + 1) + c(l)));
-                    eb[l] = cat[l];   // enc_l's output lives in the skip part of cat[l]
+                eb[l] = dalloc<uint16_t>(P * c(l));
+                if (l < kLevels - 1) {
                     da[l] = dalloc<uint16_t>(P * c(l));
                     db[l] = dalloc<uint16_t>(P * c(l));
-                    g_cat[l] = dalloc<float>(P * (c(l + 1) + c(l)));
+                    g_skip[l] = dalloc<float>(P * c(l));
                 }
                 if (l > 0) {
                     pool[l] = dalloc<uint16_t>(P * c(l - 1));
                     g_pool[l] = dalloc<float>(P * c(l - 1));
                 }
-                const int zmax = l < kLevels - 1 ? c(l + 1) + c(l) : c(l);
-                dz[l] = dalloc<uint16_t>(P * std::max(zmax, l == 0 ? cout : 0));
-                g_a[l] = dalloc<float>(P * c(l));
-                g_b[l] = dalloc<float>(P * c(l));
-                g_eb[l] = dalloc<float>(P * c(l));
+                for (auto &z : dz[l]) z = dalloc<uint16_t>(P * std::max(c(l), l == 0 ? cout : 0));
             }
-            out = dalloc<float>(pl(0) * cout);
-            g_out = dalloc<float>(pl(0) * cout);
             init(seed);
         } catch (...) {
             release();
@@ -873,44 +802,50 @@ struct UNet {
     }
 
     // ---- launch helpers with the shape checks the kernels rely on ----
-    template <bool RELU, bool OUT_F32>
-    void conv_fwd(const uint16_t *x, int xs, int xo, int cin, const uint16_t *w, const float *bias, void *y, int ys,
-                  int yo, int co, int l) {
-        if (cin % 16 || xs % 4 || xo % 4 || ys % 4 || yo % 4 || xo + cin > xs || yo + co > ys || co % 16)
-            throw Error(LLGMI_ERR_INVALID, "internal: convolution shape");
-        const int64_t P = pl(l);
-        if (xs % 8 == 0 && xo % 8 == 0 && tile_conv_enabled()) {
-            // spatial tiles of 8 rows, or 4 where 8 would leave the GPU short of blocks
-            const int nt = co % 64 == 0 ? 4 : co % 48 == 0 ? 3 : co % 32 == 0 ? 2 : 1;
-            const int64_t tiles8 = (int64_t)B * ((hl(l) + 7) / 8) * ((wl(l) + kTileW - 1) / kTileW);
-            const bool th8 = tiles8 * (co / (16 * nt)) >= 1024;
-            auto go = [&](auto thc, auto ntc) {
-                constexpr int TH = decltype(thc)::value, NT = decltype(ntc)::value;
-                launch_conv_tile<TH, NT, RELU, OUT_F32>(x, xs, xo, cin, w, bias, y, ys, yo, co, l);
-            };
-            using I8 = std::integral_constant<int, 8>;
-            using I4 = std::integral_constant<int, 4>;
-            switch (nt) {
-                case 4: th8 ? go(I8{}, std::integral_constant<int, 4>{}) : go(I4{}, std::integral_constant<int, 4>{}); break;
-                case 3: th8 ? go(I8{}, std::integral_constant<int, 3>{}) : go(I4{}, std::integral_constant<int, 3>{}); break;
-                case 2: th8 ? go(I8{}, std::integral_constant<int, 2>{}) : go(I4{}, std::integral_constant<int, 2>{}); break;
-                default: th8 ? go(I8{}, std::integral_constant<int, 1>{}) : go(I4{}, std::integral_constant<int, 1>{}); break;
-            }
-            return;
-        }
-        if (P >= kWideTileMinPixels) launch_conv<4, RELU, OUT_F32>(x, xs, xo, cin, w, bias, y, ys, yo, co, l);
-        else launch_conv<2, RELU, OUT_F32>(x, xs, xo, cin, w, bias, y, ys, yo, co, l);
+    static ConvSrc dense(const uint16_t *x, int c) { return {nullptr, 0, x, c}; }
+    static void check_src(const ConvSrc &s, int cin) {
+        if (cin % 16 || s.lo_c + s.hi_c != cin || s.lo_c % kKC) throw Error(LLGMI_ERR_INVALID, "internal: convolution input");
     }
-    // LLGMI_UNET_TILE=0 runs every convolution with k_conv3x3 (the pixel-row kernel)
-    static bool tile_conv_enabled() {
+
+    template <int EPI, bool RELU>
+    void conv3(ConvSrc src, int cin, const uint16_t *w, const float *bias, const ConvEpi &ep, int co, int l) {
+        check_src(src, cin);
+        // output channels per block: a divisor of the upsampled part too
+        int nt = co % 32 == 0 ? 2 : co % 48 == 0 ? 3 : 1;
+        if (EPI == EPI_CAT && ep.up_c % (16 * nt)) nt = 1;
+        if (co % (16 * nt) || (EPI == EPI_CAT && ep.up_c % (16 * nt)))
+            throw Error(LLGMI_ERR_INVALID, "internal: convolution shape");
+        if ((ep.pool || EPI == EPI_CAT) && (hl(l) % 2 || wl(l) % 2)) throw Error(LLGMI_ERR_INVALID, "internal: odd plane");
+        // Pixel tile: the largest that gives two blocks to every CU twice over;
+        // 16 x 32 reads least per product, but on narrow planes its padding
+        // (columns past the image) costs more than that.  LLGMI_UNET_TILE=0
+        // takes the smallest everywhere.
+        auto tiles = [&](int th, int tw) {
+            return (int64_t)B * ((hl(l) + th - 1) / th) * ((wl(l) + 16 * tw - 1) / (16 * tw));
+        };
+        const int64_t groups = co / (16 * nt);
+        const bool wide = nt < 3 && tiles(16, 2) * groups >= 1024 && 10 * 2 * tiles(16, 2) <= 11 * tiles(16, 1);
+        const bool tall = tiles(16, 1) * groups >= 512;
+        auto go = [&](auto ntc) {
+            constexpr int NT = decltype(ntc)::value;
+            if (!large_tiles()) launch_conv<8, 1, NT, EPI, RELU>(src, cin, w, bias, ep, co, l);
+            else if (wide) {
+                if constexpr (NT < 3) launch_conv<16, 2, NT, EPI, RELU>(src, cin, w, bias, ep, co, l);
+            } else if (tall) launch_conv<16, 1, NT, EPI, RELU>(src, cin, w, bias, ep, co, l);
+            else launch_conv<8, 1, NT, EPI, RELU>(src, cin, w, bias, ep, co, l);
+        };
+        if (nt == 3) go(std::integral_constant<int, 3>{});
+        else if (nt == 2) go(std::integral_constant<int, 2>{});
+        else go(std::integral_constant<int, 1>{});
+    }
+    static bool large_tiles() {
         const char *e = std::getenv("LLGMI_UNET_TILE");
         return !(e && e[0] == '0');
     }
-    template <int TH, int NT, bool RELU, bool OUT_F32>
-    void launch_conv_tile(const uint16_t *x, int xs, int xo, int cin, const uint16_t *w, const float *bias, void *y,
-                          int ys, int yo, int co, int l) {
-        constexpr size_t lds = conv_tile_lds<TH, NT>();
-        auto kern = k_conv3x3_tile<TH, NT, RELU, OUT_F32>;
+    template <int TH, int TW, int NT, int EPI, bool RELU>
+    void launch_conv(ConvSrc src, int cin, const uint16_t *w, const float *bias, const ConvEpi &ep, int co, int l) {
+        constexpr size_t lds = ConvShape<TH, TW, NT>::LDS;
+        auto kern = k_conv3x3<TH, TW, NT, EPI, RELU>;
         {
             // the LDS attribute is set once per kernel and device
             static std::mutex mu;
@@ -923,37 +858,35 @@ struct UNet {
                 done.insert(dev);
             }
         }
-        const int ntx = (wl(l) + kTileW - 1) / kTileW, nty = (hl(l) + TH - 1) / TH;
-        const dim3 grid((unsigned)(ntx * nty * B), (unsigned)(co / (16 * NT)));
-        hipLaunchKernelGGL(kern, grid, dim3(256), lds, stream, x, xs, xo, cin, w, bias, y, ys, yo, co, B, hl(l), wl(l));
+        const int ntile = ((wl(l) + 16 * TW - 1) / (16 * TW)) * ((hl(l) + TH - 1) / TH) * B, groups = co / (16 * NT);
+        // one-chunk layers run several tiles per block (weights stay in LDS)
+        const int nb = cin <= kKC ? std::min(ntile, std::max(1, 1024 / groups)) : ntile;
+        hipLaunchKernelGGL(kern, dim3((unsigned)nb, (unsigned)groups), dim3(256), lds, stream, src, cin, w, bias, ep, co,
+                           B, hl(l), wl(l));
         LLGMI_LAUNCH_CHECK();
     }
-    template <int MT, bool RELU, bool OUT_F32>
-    void launch_conv(const uint16_t *x, int xs, int xo, int cin, const uint16_t *w, const float *bias, void *y,
-                     int ys, int yo, int co, int l) {
-        const int64_t P = pl(l);
-        const int gx = (int)((P + 64 * MT - 1) / (64 * MT));
-        auto lds = [&](int nt) { return (size_t)16 * nt * (cin + 8) * sizeof(uint16_t); };
-        if (lds(co % 64 == 0 ? 4 : co % 32 == 0 ? 2 : 1) > kConvLdsMax)
-            throw Error(LLGMI_ERR_INVALID, "internal: convolution weight slice exceeds LDS");
-        if (co % 64 == 0)
-            hipLaunchKernelGGL((k_conv3x3<MT, 4, RELU, OUT_F32>), dim3(gx, co / 64), dim3(256), lds(4), stream, x,
-                               xs, xo, cin, w, bias, y, ys, yo, co, B, hl(l), wl(l));
-        else if (co % 32 == 0)
-            hipLaunchKernelGGL((k_conv3x3<MT, 2, RELU, OUT_F32>), dim3(gx, co / 32), dim3(256), lds(2), stream, x,
-                               xs, xo, cin, w, bias, y, ys, yo, co, B, hl(l), wl(l));
-        else
-            hipLaunchKernelGGL((k_conv3x3<MT, 1, RELU, OUT_F32>), dim3(gx, co / 16), dim3(256), lds(1), stream, x,
-                               xs, xo, cin, w, bias, y, ys, yo, co, B, hl(l), wl(l));
-        LLGMI_LAUNCH_CHECK();
+    // forward of a hidden layer: bf16 relu(conv + bias) to y, and its average pool
+    void act(ConvSrc src, const UNetConv &cv, uint16_t *y, int l, uint16_t *pooled = nullptr) {
+        ConvEpi ep;
+        ep.y = y;
+        ep.pool = pooled;
+        conv3<EPI_ACT, true>(src, cv.cin, cv.wf, d_p + cv.b_off, ep, cv.cout, l);
     }
-    void wgrad(const uint16_t *dzp, int co, const uint16_t *x, int xs, int xo, int ci, const UNetConv &cv, int l) {
-        if (co % 16 || ci % 16 || xo + ci > xs || co != cv.cout || ci != cv.cin)
-            throw Error(LLGMI_ERR_INVALID, "internal: weight-gradient shape");
+    // data gradient of cv from dz, masked by the activation it flows into
+    void dgrad(const uint16_t *dzp, const UNetConv &cv, const uint16_t *mask, uint16_t *y, int l) {
+        ConvEpi ep;
+        ep.y = y;
+        ep.mask = mask;
+        conv3<EPI_MASK, false>(dense(dzp, cv.cout), cv.cout, cv.wb, nullptr, ep, cv.cin, l);
+    }
+    void wgrad(const uint16_t *dzp, ConvSrc src, const UNetConv &cv, int l) {
+        const int co = cv.cout, ci = cv.cin;
+        check_src(src, ci);
+        if (co % 16) throw Error(LLGMI_ERR_INVALID, "internal: weight-gradient shape");
         const int mt = wgrad_mt(co), nt = wgrad_nt(co, ci);
         const dim3 grid((unsigned)wgrad_split(co, ci, l), (unsigned)((co / (16 * mt)) * (ci / (16 * nt))));
         auto go = [&](auto kern) {
-            hipLaunchKernelGGL(kern, grid, dim3(256), 0, stream, dzp, co, x, xs, xo, ci, d_part, B, hl(l), wl(l));
+            hipLaunchKernelGGL(kern, grid, dim3(256), 0, stream, dzp, co, src, ci, d_part, B, hl(l), wl(l));
         };
         if (mt == 3) go(k_conv3x3_wgrad<3, 1>);
         else if (mt == 2) nt == 2 ? go(k_conv3x3_wgrad<2, 2>) : go(k_conv3x3_wgrad<2, 1>);
@@ -983,97 +916,77 @@ struct UNet {
     const UNetConv &head() const { return conv.back(); }
     static int level_of(int k) { return k < 2 * kLevels ? k / 2 : k == 4 * kLevels - 2 ? 0 : kLevels - 2 - (k - 2 * kLevels) / 2; }
 
-    void forward(const uint16_t *x) {
+    // decoder l's input: the upsampled level below and enc_l's output
+    ConvSrc cat(int l) const { return {l == kLevels - 2 ? eb[l + 1] : db[l + 1], c(l + 1), eb[l], c(l)}; }
+
+    // every layer but the head
+    void trunk(const uint16_t *x) {
         for (int l = 0; l < kLevels; ++l) {
-            const uint16_t *src = l == 0 ? x : pool[l];
-            const int cs = l == 0 ? 16 : c(l - 1);
-            if (l > 0) {
-                const int cprev = c(l - 1);
-                const int ps = l - 1 < kLevels - 1 ? c(l) + cprev : cprev;   // eb[l-1] stride
-                const int po = l - 1 < kLevels - 1 ? c(l) : 0;
-                if (cprev % 8 == 0 && ps % 8 == 0 && po % 8 == 0)
-                    hipLaunchKernelGGL(k_pool2_v8, dim3(grid_of(pl(l) * cprev / 8)), dim3(kNT), 0, stream, eb[l - 1],
-                                       ps, po, cprev, pool[l], B, hl(l - 1), wl(l - 1));
-                else
-                    hipLaunchKernelGGL(k_pool2, dim3(grid_of(pl(l) * cprev)), dim3(kNT), 0, stream, eb[l - 1], ps, po,
-                                       cprev, pool[l], B, hl(l - 1), wl(l - 1));
-            }
-            conv_fwd<true, false>(src, cs, 0, cs, enc(l, 0).wf, d_p + enc(l, 0).b_off, ea[l], c(l), 0, c(l), l);
-            const int es = l < kLevels - 1 ? c(l + 1) + c(l) : c(l), eo = l < kLevels - 1 ? c(l + 1) : 0;
-            conv_fwd<true, false>(ea[l], c(l), 0, c(l), enc(l, 1).wf, d_p + enc(l, 1).b_off, eb[l], es, eo, c(l), l);
+            act(l == 0 ? dense(x, 16) : dense(pool[l], c(l - 1)), enc(l, 0), ea[l], l);
+            act(dense(ea[l], c(l)), enc(l, 1), eb[l], l, l + 1 < kLevels ? pool[l + 1] : nullptr);
         }
         for (int l = kLevels - 2; l >= 0; --l) {
-            const uint16_t *below = l == kLevels - 2 ? eb[l + 1] : db[l + 1];
-            const int cs = c(l + 1) + c(l);
-            if (c(l + 1) % 8 == 0 && cs % 8 == 0)
-                hipLaunchKernelGGL(k_up2_v8, dim3(grid_of(pl(l) * c(l + 1) / 8)), dim3(kNT), 0, stream, below,
-                                   c(l + 1), cat[l], cs, 0, B, hl(l), wl(l));
-            else
-                hipLaunchKernelGGL(k_up2, dim3(grid_of(pl(l) * c(l + 1))), dim3(kNT), 0, stream, below, c(l + 1), cat[l],
-                                   cs, 0, B, hl(l), wl(l));
-            conv_fwd<true, false>(cat[l], cs, 0, cs, dec(l, 0).wf, d_p + dec(l, 0).b_off, da[l], c(l), 0, c(l), l);
-            conv_fwd<true, false>(da[l], c(l), 0, c(l), dec(l, 1).wf, d_p + dec(l, 1).b_off, db[l], c(l), 0, c(l), l);
+            act(cat(l), dec(l, 0), da[l], l);
+            act(dense(da[l], c(l)), dec(l, 1), db[l], l);
         }
-        conv_fwd<false, true>(db[0], c(0), 0, c(0), head().wf, d_p + head().b_off, out, cout, 0, cout, 0);
-        LLGMI_LAUNCH_CHECK();
     }
-
-    // relu'(y) applied to g (dense C), cast to bf16 into dz[l]
-    void relu_bwd(const float *g, const uint16_t *y, int ys, int yo, int C, int l) {
-        if (C % 8 == 0 && (!y || (ys % 8 == 0 && yo % 8 == 0)))
-            hipLaunchKernelGGL(k_relu_bwd_v8, dim3(grid_of(pl(l) * C / 8)), dim3(kNT), 0, stream, g, y, ys, yo, C, dz[l],
-                               pl(l));
-        else
-            hipLaunchKernelGGL(k_relu_bwd, dim3(grid_of(pl(l) * C)), dim3(kNT), 0, stream, g, y, ys, yo, C, dz[l],
-                               pl(l));
+    void forward(const uint16_t *x, float *y) {
+        trunk(x);
+        ConvEpi ep;
+        ep.yf = y;
+        conv3<EPI_F32, false>(dense(db[0], c(0)), c(0), head().wf, d_p + head().b_off, ep, cout, 0);
     }
 
     // gradient of the loss w.r.t. every parameter into d_g (overwritten)
     double loss_grad(const uint16_t *x, const uint16_t *tgt) {
-        forward(x);
         LLGMI_HIP(hipMemsetAsync(d_loss, 0, sizeof(double), stream));
-        const double count = (double)B * std::min(wv, W) * std::min(hv, H) * cout_real;
-        hipLaunchKernelGGL(k_mse, dim3(grid_of(pl(0) * cout)), dim3(kNT), 0, stream, out, tgt, cout, cout_real, wv,
-                           hv, B, H, W, 1.0 / count, g_out, d_loss);
-        LLGMI_HIP(hipMemcpyAsync(h_loss, d_loss, sizeof(double), hipMemcpyDeviceToHost, stream));
-        // head
-        relu_bwd(g_out, nullptr, 0, 0, cout, 0);
-        wgrad(dz[0], cout, db[0], c(0), 0, c(0), head(), 0);
-        conv_fwd<false, true>(dz[0], cout, 0, cout, head().wb, nullptr, g_b[0], c(0), 0, c(0), 0);
-        // decoders, top level first
-        for (int l = 0; l <= kLevels - 2; ++l) {
-            const int cs = c(l + 1) + c(l);
-            relu_bwd(g_b[l], db[l], c(l), 0, c(l), l);
-            wgrad(dz[l], c(l), da[l], c(l), 0, c(l), dec(l, 1), l);
-            conv_fwd<false, true>(dz[l], c(l), 0, c(l), dec(l, 1).wb, nullptr, g_a[l], c(l), 0, c(l), l);
-            relu_bwd(g_a[l], da[l], c(l), 0, c(l), l);
-            wgrad(dz[l], c(l), cat[l], cs, 0, cs, dec(l, 0), l);
-            conv_fwd<false, true>(dz[l], c(l), 0, c(l), dec(l, 0).wb, nullptr, g_cat[l], cs, 0, cs, l);
-            // up part -> gradient of the level below's decoder output (or the bottleneck)
-            float *gbelow = l + 1 == kLevels - 1 ? g_eb[l + 1] : g_b[l + 1];
-            hipLaunchKernelGGL(k_up2_bwd, dim3(grid_of(pl(l + 1) * c(l + 1))), dim3(kNT), 0, stream, g_cat[l], cs, 0,
-                               c(l + 1), gbelow, B, hl(l), wl(l));
-            // skip part -> gradient of enc_l's output (the pool gradient is added later)
-            hipLaunchKernelGGL(k_slice_copy, dim3(grid_of(pl(l) * c(l))), dim3(kNT), 0, stream, g_cat[l], cs, c(l + 1),
-                               c(l), g_eb[l], pl(l));
+        trunk(x);
+        {
+            // head with the loss and its gradient
+            ConvEpi ep;
+            ep.y = dz[0][0];
+            ep.tgt = tgt;
+            ep.cv = cout_real;
+            ep.wv = wv;
+            ep.hv = hv;
+            ep.inv_count = 1.0 / ((double)B * std::min(wv, W) * std::min(hv, H) * cout_real);
+            ep.loss = d_loss;
+            conv3<EPI_MSE, false>(dense(db[0], c(0)), c(0), head().wf, d_p + head().b_off, ep, cout, 0);
         }
-        // encoders, bottom level first
+        LLGMI_HIP(hipMemcpyAsync(h_loss, d_loss, sizeof(double), hipMemcpyDeviceToHost, stream));
+        wgrad(dz[0][0], dense(db[0], c(0)), head(), 0);
+        dgrad(dz[0][0], head(), db[0], dz[0][1], 0);
+        // decoders, top level first; dz[l][1] holds the gradient of dec_l's output
+        for (int l = 0; l <= kLevels - 2; ++l) {
+            wgrad(dz[l][1], dense(da[l], c(l)), dec(l, 1), l);
+            dgrad(dz[l][1], dec(l, 1), da[l], dz[l][0], l);
+            wgrad(dz[l][0], cat(l), dec(l, 0), l);
+            // up part: masked gradient of the level below's output; skip part: to be joined by the pool's
+            ConvEpi ep;
+            ep.y = dz[l + 1][1];
+            ep.mask = cat(l).lo;
+            ep.up_c = c(l + 1);
+            ep.yf = g_skip[l];
+            conv3<EPI_CAT, false>(dense(dz[l][0], c(l)), c(l), dec(l, 0).wb, nullptr, ep, dec(l, 0).cin, l);
+        }
+        // encoders, bottom level first; dz[l][1] holds the gradient of enc_l's output
         for (int l = kLevels - 1; l >= 0; --l) {
-            const int es = l < kLevels - 1 ? c(l + 1) + c(l) : c(l), eo = l < kLevels - 1 ? c(l + 1) : 0;
-            relu_bwd(g_eb[l], eb[l], es, eo, c(l), l);
-            wgrad(dz[l], c(l), ea[l], c(l), 0, c(l), enc(l, 1), l);
-            conv_fwd<false, true>(dz[l], c(l), 0, c(l), enc(l, 1).wb, nullptr, g_a[l], c(l), 0, c(l), l);
-            relu_bwd(g_a[l], ea[l], c(l), 0, c(l), l);
+            if (l < kLevels - 1) {
+                hipLaunchKernelGGL(k_skip_pool_relu, dim3(grid_of(pl(l) * c(l) / 8)), dim3(kNT), 0, stream, g_skip[l],
+                                   g_pool[l + 1], eb[l], c(l), dz[l][1], B, hl(l), wl(l));
+                LLGMI_LAUNCH_CHECK();
+            }
+            wgrad(dz[l][1], dense(ea[l], c(l)), enc(l, 1), l);
+            dgrad(dz[l][1], enc(l, 1), ea[l], dz[l][0], l);
             if (l == 0) {
-                wgrad(dz[0], c(0), x, 16, 0, 16, enc(0, 0), 0);
+                wgrad(dz[0][0], dense(x, 16), enc(0, 0), 0);
             } else {
-                wgrad(dz[l], c(l), pool[l], c(l - 1), 0, c(l - 1), enc(l, 0), l);
-                conv_fwd<false, true>(dz[l], c(l), 0, c(l), enc(l, 0).wb, nullptr, g_pool[l], c(l - 1), 0, c(l - 1), l);
-                hipLaunchKernelGGL(k_pool2_bwd, dim3(grid_of(pl(l - 1) * c(l - 1))), dim3(kNT), 0, stream, g_pool[l],
-                                   c(l - 1), g_eb[l - 1], B, hl(l - 1), wl(l - 1));
+                wgrad(dz[l][0], dense(pool[l], c(l - 1)), enc(l, 0), l);
+                ConvEpi ep;
+                ep.yf = g_pool[l];
+                conv3<EPI_F32, false>(dense(dz[l][0], c(l)), c(l), enc(l, 0).wb, nullptr, ep, c(l - 1), l);
             }
         }
-        LLGMI_LAUNCH_CHECK();
         LLGMI_HIP(hipStreamSynchronize(stream));
         return *h_loss;
     }
@@ -1203,9 +1116,7 @@ int llgmi_ws_forward(llgmi_ws *ws, const uint16_t *x_dev, float *y_dev) {
     return ws_guard(ws, [&](UNet &u) {
         need(x_dev, x_bytes(u), "x");
         need(y_dev, y_bytes(u), "y");
-        u.forward(x_dev);
-        const int64_t n = u.pl(0) * u.cout;
-        LLGMI_HIP(hipMemcpyAsync(y_dev, u.out, sizeof(float) * (size_t)n, hipMemcpyDeviceToDevice, u.stream));
+        u.forward(x_dev, y_dev);
         LLGMI_HIP(hipStreamSynchronize(u.stream));
     });
 }
