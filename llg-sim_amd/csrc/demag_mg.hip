@@ -71,6 +71,55 @@ __device__ __forceinline__ int64_t idx3(int i, int j, int k, int nx, int ny) {
 
 __device__ __forceinline__ int clampi(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); }
 
+// a / d for a divisor fixed over a launch, correctly rounded: r = RN(1 / d) is
+// formed once on the host; q0 = a r is within two ulp, the first correction
+// makes it faithful, and the second, whose remainder is exact, gives RN(a / d)
+// (Markstein 1990, "Computation of elementary functions on the IBM RISC System
+// / 6000 processor", theorem on division with a correctly rounded reciprocal).
+// The theorem excludes a divisor whose mantissa is all ones (the host then sets
+// ok = 0); numerators beyond 2^900 and infinities take the division itself.  A
+// numerator below 2^-900 may be off in the last place of its quotient, where the
+// remainders underflow.  Five multiply-adds against about twelve instructions
+// and a quarter-rate reciprocal.
+struct ExactDiv {
+    double d, r;
+    int ok;
+};
+inline ExactDiv exact_div(double d) {
+    uint64_t u;
+    std::memcpy(&u, &d, 8);
+    const double a = std::fabs(d);
+    ExactDiv e{d, 1.0 / d, 0};
+    e.ok = a > 0x1p-100 && a < 0x1p100 && (u & 0xfffffffffffffull) != 0xfffffffffffffull;
+    return e;
+}
+// a[i] / d for N independent quotients side by side, with one test for all
+template <int N>
+__device__ __forceinline__ void div_by(double (&a)[N], const ExactDiv &e) {
+    double q[N], m = 0.0;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        m = fmax(m, fabs(a[i]));
+        const double q0 = a[i] * e.r;
+        const double q1 = __builtin_fma(__builtin_fma(-q0, e.d, a[i]), e.r, q0);
+        q[i] = __builtin_fma(__builtin_fma(-q1, e.d, a[i]), e.r, q1);
+    }
+    if (!e.ok || m > 0x1p900) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) q[i] = a[i] / e.d;
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) a[i] = q[i];
+}
+
+// The value, hidden from the optimiser: addresses formed from it are recomputed
+// where they are used instead of being kept, one register pair per access, over
+// an unrolled loop.
+__device__ __forceinline__ uint32_t opaque(uint32_t v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
 // offdiag_sum_at (mg_kernels.rs:72-94)
 __device__ __forceinline__ double offdiag(const double *__restrict__ phi, int nx, int ny, int nz, int i,
                                           int j, int k, const DevStencil *__restrict__ st) {
@@ -200,7 +249,7 @@ __global__ void __launch_bounds__(kNT) k_mg_rhs(const T *__restrict__ m, int64_t
 // needed.  Thread -> (interior row, h), i = first cell of the colour + 2h.
 __global__ void __launch_bounds__(kNT) k_mg_rb(double *__restrict__ phi, const double *__restrict__ rhs,
                                                int nx, int ny, int nz, double sx, double sy, double sz,
-                                               double denom, double omega, int color) {
+                                               ExactDiv denom, double omega, int color) {
     const int H = (nx - 1) / 2;
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t rows = (int64_t)(ny - 2) * (nz - 2);
@@ -215,197 +264,250 @@ __global__ void __launch_bounds__(kNT) k_mg_rb(double *__restrict__ phi, const d
     const int64_t plane = (int64_t)nx * ny;
     const double off = sx * (phi[id - 1] + phi[id + 1]) + sy * (phi[id - nx] + phi[id + nx]) +
                        sz * (phi[id - plane] + phi[id + plane]);
-    const double pn = (off - rhs[id]) / denom;
+    double pn[1] = {off - rhs[id]};
+    div_by(pn, denom);
     const double po = phi[id];
-    phi[id] = po + omega * (pn - po);
+    phi[id] = po + omega * (pn[0] - po);
 }
 
-// One full red-black SOR sweep (colour 0, then colour 1) from A into B.
-// The colour-1 update reads the new colour-0 values and the old own value,
-// the colour-0 update only old values, so with separate input and output
-// buffers the sweep is the reference's in-place pair of half-sweeps exactly.
-// A block owns an RBX x RBY tile of interior (i, j) columns and a chunk of
-// RBZ planes and marches up k.  Two rings in LDS: the old values A of four
-// planes on the tile plus a two-cell halo (each plane read from HBM once,
-// when the march reaches it), and the new colour-0 values of planes k-1, k,
-// k+1 on the tile plus a one-cell halo (halo cells and the plane below the
-// chunk recomputed, boundary cells keep their value).  rbz = planes per
-// chunk (z-chunks add blocks at the cost of recomputed planes).
-constexpr int RBX = 32, RBY = 8, RBW = RBX + 2, RBH = RBY + 2, RAW = RBX + 4, RAH = RBY + 4;
-__global__ void __launch_bounds__(RBX * RBY) k_mg_rb_sweep(const double *__restrict__ A, double *__restrict__ B,
-                                                       const double *__restrict__ rhs, int nx, int ny,
-                                                       int nz, double sx, double sy, double sz, double denom,
-                                                       double omega, int rbz) {
-    __shared__ double red[3][RBH][RBW];
-    __shared__ double av[4][RAH][RAW];   // A on plane p in slot p % 4, origin (i0 - 2, j0 - 2)
-    const int tid = threadIdx.x;
-    const int i0 = 1 + (int)blockIdx.x * RBX, j0 = 1 + (int)blockIdx.y * RBY;
-    const int kb = 1 + (int)blockIdx.z * rbz, ke = min(nz - 2, kb + rbz - 1);
-    auto load = [&](int k) {
-        if (k < 0 || k >= nz) return;
-        double(*a)[RAW] = av[k & 3];
-        for (int q = tid; q < RAH * RAW; q += RBX * RBY) {
-            const int hj = q / RAW, hi = q - hj * RAW;
-            const int i = i0 - 2 + hi, j = j0 - 2 + hj;
-            a[hj][hi] = (i >= 0 && i < nx && j >= 0 && j < ny) ? A[idx3(i, j, k, nx, ny)] : 0.0;
-        }
-    };
-    // new colour-0 value at an even cell (i, j, k), or the unchanged value of a
-    // boundary cell; A from the LDS ring (planes k-1, k, k+1 loaded)
-    auto red_new = [&](int i, int j, int k) -> double {
-        const int hi = i - (i0 - 2), hj = j - (j0 - 2);
-        const double(*ac)[RAW] = av[k & 3];
-        if (i <= 0 || i >= nx - 1 || j <= 0 || j >= ny - 1 || k <= 0 || k >= nz - 1) return ac[hj][hi];
-        const double(*am)[RAW] = av[(k - 1) & 3];
-        const double(*ap)[RAW] = av[(k + 1) & 3];
-        const double off = sx * (ac[hj][hi - 1] + ac[hj][hi + 1]) + sy * (ac[hj - 1][hi] + ac[hj + 1][hi]) +
-                           sz * (am[hj][hi] + ap[hj][hi]);
-        const double pn = (off - rhs[idx3(i, j, k, nx, ny)]) / denom;
-        const double po = ac[hj][hi];
-        return po + omega * (pn - po);
-    };
-    // only even-parity positions are ever read by the colour-1 update: the
-    // in-plane and vertical neighbours of an odd cell are even
-    auto fill = [&](int slot, int k) {
-        for (int q = tid; q < (RBW / 2) * RBH; q += RBX * RBY) {
-            const int hj = q / (RBW / 2);
-            const int hi = 2 * (q % (RBW / 2)) + ((i0 + j0 + hj + k) & 1);
-            const int i = i0 - 1 + hi, j = j0 - 1 + hj;
-            red[slot][hj][hi] = (i < nx && j < ny) ? red_new(i, j, k) : 0.0;
-        }
-    };
-    for (int k = kb - 2; k <= kb + 1; ++k) load(k);
-    __syncthreads();
-    fill((kb - 1) % 3, kb - 1);
-    fill(kb % 3, kb);
-    const int ti = tid % RBX, tj = tid / RBX;
-    const int i = i0 + ti, j = j0 + tj;
-    const bool inside = i <= nx - 2 && j <= ny - 2;
-    // cells that never change: boundary columns and rows next to this tile
-    // (the planes of this chunk, plus the bottom / top plane for the first /
-    // last chunk) and the bottom / top planes under the tile
-    if (inside) {
-        const int klo = kb == 1 ? 0 : kb, khi = ke == nz - 2 ? nz - 1 : ke;
-        auto keep = [&](int a, int c) {
-            for (int k = klo; k <= khi; ++k) B[idx3(a, c, k, nx, ny)] = A[idx3(a, c, k, nx, ny)];
-        };
-        if (i == 1) keep(0, j);
-        if (i == nx - 2) keep(nx - 1, j);
-        if (j == 1) keep(i, 0);
-        if (j == ny - 2) keep(i, ny - 1);
-        if (i == 1 && j == 1) keep(0, 0);
-        if (i == nx - 2 && j == 1) keep(nx - 1, 0);
-        if (i == 1 && j == ny - 2) keep(0, ny - 1);
-        if (i == nx - 2 && j == ny - 2) keep(nx - 1, ny - 1);
-        if (kb == 1) B[idx3(i, j, 0, nx, ny)] = av[0][tj + 2][ti + 2];
-        if (ke == nz - 2) B[idx3(i, j, nz - 1, nx, ny)] = A[idx3(i, j, nz - 1, nx, ny)];
+// Two red-black SOR sweeps (colours 0, 1, 0, 1) from A into B in one pass over
+// memory.  A block owns a (BX-8) x (BY-8) tile of columns plus a four-cell
+// halo, one thread per pair of columns x = 2c, 2c+1, and marches up z.  The four
+// half-sweeps follow each other through the planes: step s updates colour 0 of
+// the first sweep on plane s and of the second on plane s-3, then (one barrier
+// later) colour 1 on planes s-1 and s-4.  A half-sweep reads only the other
+// colour, and with this lag every value it reads is the one the in-place pair
+// of half-sweeps would read, so the result is that of the separate sweeps bit
+// for bit; halo cells go stale one ring per half-sweep and are not written.
+//
+// A thread keeps its two columns of the eight live planes in registers: the
+// cell itself, its vertical neighbours and one horizontal neighbour come from
+// there, three neighbours from LDS, which holds the planes with a row's even and
+// odd cells apart ([plane & 7][row][x & 1][x / 2]), so the lanes of a wave read
+// consecutive words.  The march is unrolled over the eight planes of the ring,
+// which makes register and LDS slots constants.
+//
+// Traffic: phi in, rhs in twice (the second time from L2), phi out once for two
+// sweeps.
+// At 524 x 524 x 36: 66 us for two sweeps (3.6 TB/s over phi, rhs and the
+// result once each), against 2 x 98 us for the earlier one-sweep march (which read phi
+// and rhs once per sweep, through a serial division per cell); 80 us without the
+// XCD order.  The 32 x 16 box at 262 x 262 x 18: 25 us against 46 us for four
+// half-sweep launches.
+template <int BX, int BY>
+__global__ void __launch_bounds__(BX *BY / 2) k_mg_rb_sweep2(const double *__restrict__ A, double *__restrict__ B,
+                                                             const double *__restrict__ rhs, int nx, int ny, int nz,
+                                                             double sx, double sy, double sz, ExactDiv denom,
+                                                             double omega) {
+    constexpr int HX = BX / 2, TX = BX - 8, TY = BY - 8, PLANE = BX * BY;
+    extern __shared__ unsigned char lds_raw[];
+    // a row before and after the planes: rows 0 and BY-1 read (and drop) their neighbours too
+    double *lds = reinterpret_cast<double *>(lds_raw) + BX;
+    const int c = threadIdx.x % HX, y = threadIdx.x / HX;
+    // neighbouring tiles (they share halo columns) on one XCD
+    const int lb = xcd_remap((int)(blockIdx.y * gridDim.x + blockIdx.x), (int)(gridDim.x * gridDim.y));
+    const int by = lb / (int)gridDim.x, bx = lb - by * (int)gridDim.x;
+    const int i0 = 1 + bx * TX, j0 = 1 + by * TY;
+    const int gi = i0 - 4 + 2 * c, gj = j0 - 4 + y;   // column 2c of the box
+    // column index 0: the one whose cells are colour 0 on even planes
+    const int q = (gi + gj) & 1;
+    const bool rowin = gj >= 0 && gj < ny, rowup = y >= 1 && y < BY - 1 && gj >= 1 && gj <= ny - 2;
+    const int ylo = by == 0 ? 0 : j0, yhi = j0 + TY > ny - 2 ? ny - 1 : j0 + TY - 1;
+    const int xlo = bx == 0 ? 0 : i0, xhi = i0 + TX > nx - 2 ? nx - 1 : i0 + TX - 1;
+    const bool rowout = gj >= ylo && gj <= yhi;
+    bool in[2], up[2], out[2];
+    int own[2], nbx[2];
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+        const int par = a ^ q, x = 2 * c + par, g = gi + par;
+        in[a] = rowin && g >= 0 && g < nx;
+        up[a] = rowup && x >= 1 && x < BX - 1 && g >= 1 && g <= nx - 2;
+        out[a] = in[a] && rowout && g >= xlo && g <= xhi;
+        own[a] = (y * 2 + par) * HX + c;
+        // the neighbours outside the pair; columns that are not updated read themselves
+        nbx[a] = !up[a] ? own[a] : par ? y * 2 * HX + c + 1 : (y * 2 + 1) * HX + c - 1;
     }
-    for (int k = kb; k <= ke; ++k) {
-        const int sm = (k - 1) % 3, sc = k % 3, sp = (k + 1) % 3;
-        load(k + 2);   // slot of plane k - 2, which no step below reads
-        __syncthreads();
-        fill(sp, k + 1);
-        __syncthreads();
-        if (inside) {
-            const int64_t id = idx3(i, j, k, nx, ny);
-            const int hi = ti + 1, hj = tj + 1;
-            if (((i + j + k) & 1) == 0) {
-                B[id] = red[sc][hj][hi];
-            } else {
-                const double off = sx * (red[sc][hj][hi - 1] + red[sc][hj][hi + 1]) +
-                                   sy * (red[sc][hj - 1][hi] + red[sc][hj + 1][hi]) +
-                                   sz * (red[sm][hj][hi] + red[sp][hj][hi]);
-                const double pn = (off - rhs[id]) / denom;
-                const double po = av[k & 3][tj + 2][ti + 2];
-                B[id] = po + omega * (pn - po);
+    const int64_t plane = (int64_t)nx * ny;
+    // byte offsets within a plane (a box has fewer than 2^31 cells on at least
+    // four planes); the plane's address is uniform
+    uint32_t at[2];
+#pragma unroll
+    for (int a = 0; a < 2; ++a) at[a] = in[a] ? ((uint32_t)gj * (uint32_t)nx + (uint32_t)(gi + (a ^ q))) * 8u : 0u;
+    auto cell = [&](const double *f, int k, int a) {
+        return reinterpret_cast<const double *>(reinterpret_cast<const char *>(f + k * plane) + opaque(at[a]));
+    };
+    double v[8][2];
+    auto fetch = [&](int k, int u) {   // phi of plane k into ring slot u
+#pragma unroll
+        for (int a = 0; a < 2; ++a) v[u][a] = in[a] && k < nz ? *cell(A, k, a) : 0.0;
+    };
+    // rhs of one column's cell on plane k, loaded a step ahead of each of its two
+    // uses (the second read finds it in L2)
+    auto fetch_r = [&](int k, int a) { return up[a] && k >= 1 && k < nz ? *cell(rhs, k, a) : 0.0; };
+    auto stage = [&](int u) {
+        lds[u * PLANE + own[0]] = v[u][0];
+        lds[u * PLANE + own[1]] = v[u][1];
+    };
+    // one cell each of column a0 on plane k0 and column a1 on plane k1 (ring
+    // slots u0, u1) with right sides r0, r1
+    auto update = [&](int k0, int u0, int a0, double r0, int k1, int u1, int a1, double r1) {
+        const int kk[2] = {k0, k1}, uu[2] = {u0, u1}, aa[2] = {a0, a1};
+        double pn[2] = {r0, r1};
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int u = uu[i], a = aa[i];
+            const double *p = lds + u * PLANE;
+            const double off = sx * (v[u][1 - a] + p[nbx[a]]) + sy * (p[own[a] - BX] + p[own[a] + BX]) +
+                               sz * (v[(u + 7) & 7][a] + v[(u + 1) & 7][a]);
+            pn[i] = off - pn[i];
+        }
+        div_by(pn, denom);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int u = uu[i], a = aa[i];
+            if (up[a] && kk[i] >= 1 && kk[i] <= nz - 2) {
+                v[u][a] += omega * (pn[i] - v[u][a]);
+                lds[u * PLANE + own[a]] = v[u][a];
             }
         }
+    };
+    fetch(0, 0);
+    fetch(1, 1);
+#pragma unroll
+    for (int u = 3; u < 8; ++u) v[u][0] = v[u][1] = 0.0;
+    stage(0);
+    stage(1);
+    fetch(2, 2);
+    double r[4] = {0.0, 0.0, 0.0, 0.0};   // right sides of a step's four updates
+    __syncthreads();
+    for (int s0 = 0; s0 < nz + 4; s0 += 8) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int s = s0 + u, e = u & 1, o = 1 - e;
+            if (s >= nz + 4) break;
+            // colour 0 of the first sweep on plane s, of the second on s - 3
+            update(s, u, e, r[0], s - 3, (u + 5) & 7, o, r[1]);
+            r[0] = fetch_r(s + 1, o);
+            r[1] = fetch_r(s - 2, e);
+            __syncthreads();
+            // colour 1: planes s - 1 and s - 4
+            update(s - 1, (u + 7) & 7, e, r[2], s - 4, (u + 4) & 7, o, r[3]);
+            r[2] = fetch_r(s, o);
+            r[3] = fetch_r(s - 3, e);
+            if (s >= 4) {   // plane s - 4 is final
+#pragma unroll
+                for (int a = 0; a < 2; ++a)
+                    if (out[a]) *const_cast<double *>(cell(B, s - 4, a)) = v[(u + 4) & 7][a];
+            }
+            stage((u + 2) & 7);
+            fetch(s + 3, (u + 3) & 7);   // the slot of plane s - 5, read for the last time above
+            __syncthreads();
+        }
     }
 }
 
-// Up to TBH red-black half-sweeps (colours alternating from `color`) in one
-// launch, for small levels (the coarsest level's 80 sweeps).  A block loads
-// an (TBT + 2 TBH)^2 x nz box of A and of rhs into LDS, updates the A box in
-// place half-sweep by half-sweep (each half-sweep leaves one more outer ring
-// stale), and writes the central TBT x TBT columns to B; after h <= TBH
-// half-sweeps those are exactly the values the in-place half-sweeps produce.
-// TBT = 10 puts the 131 x 131 coarsest level of the 512^2 film in 169 blocks
-// (one per CU, one round on 256 CUs, 97 KB of LDS each); measured against 8,
-// 12 and 16 it gives the shortest launches (fewer cells per block, no second
-// round of blocks).
-constexpr int TBT = 10, TBH = 8, TBW = TBT + 2 * TBH, TB_MAXZ = 9, TB_NT = 1024;
-__device__ __forceinline__ int tb_at(int k, int hj, int hi) { return (k * TBW + hj) * TBW + hi; }
+// `nhalf` red-black half-sweeps (colours alternating from `color`) in one
+// launch, for small levels of at most TB_MAXZ planes (the coarsest level's 80
+// sweeps).  A block holds a TBW x TBW x nz box, its central tile T columns wide,
+// halo (TBW - T) / 2 >= nhalf; each half-sweep leaves one more outer ring stale,
+// and the tile is exact at the end.  One thread per pair of columns: their
+// cells and rhs stay in registers (of a pair, one column's even and the other's
+// odd planes are of one colour, so a half-sweep updates seven cells per thread
+// at fixed registers), and three neighbours of a cell come from LDS, laid out as
+// above.
+// The level has few cells, so a launch lasts as long as one block: the host
+// takes the narrowest tile (the most half-sweeps per launch) whose blocks still
+// find a CU each.
+// 131 x 131 x 9: 15.5 us for 11 half-sweeps (15 launches per 80 sweeps) against
+// 15.5 us for 8 (20 launches) with a box read from LDS throughout, divided by the
+// instruction sequence, and updated in full at every half-sweep.
+constexpr int TBW = 32, TB_MAXZ = 9, TB_NT = TBW * TBW / 2;
+template <bool FULL>   // nz == TB_MAXZ
 __global__ void __launch_bounds__(TB_NT) k_mg_rb_tb(const double *__restrict__ A, double *__restrict__ B,
                                                     const double *__restrict__ rhs, int nx, int ny, int nz,
-                                                    double sx, double sy, double sz, double denom,
-                                                    double omega, int color, int nhalf) {
+                                                    double sx, double sy, double sz, ExactDiv denom,
+                                                    double omega, int color, int nhalf, int T) {
+    constexpr int HX = TBW / 2, PLANE = TBW * TBW;
     extern __shared__ unsigned char lds_raw[];
-    const int nbox = nz * TBW * TBW;
-    double *box = reinterpret_cast<double *>(lds_raw);   // A, [nz][TBW][TBW]
-    double *rb = box + nbox;                               // rhs, same layout
-    const int tid = threadIdx.x;
-    const int i0 = 1 + (int)blockIdx.x * TBT, j0 = 1 + (int)blockIdx.y * TBT;
-    const int ib = i0 - TBH, jb = j0 - TBH;   // global index of box column 0
-    {
-        // all global loads of this thread first, then the LDS stores
-        constexpr int PER = (TB_MAXZ * TBW * TBW + TB_NT - 1) / TB_NT;
-        double va[PER], vr[PER];
+    double *lds = reinterpret_cast<double *>(lds_raw);   // [TB_MAXZ][TBW][2][HX]
+    const int c = threadIdx.x % HX, y = threadIdx.x / HX, halo = (TBW - T) / 2;
+    const int i0 = 1 + (int)blockIdx.x * T, j0 = 1 + (int)blockIdx.y * T;
+    const int gi = i0 - halo + 2 * c, gj = j0 - halo + y;
+    const int q = (gi + gj) & 1;   // column index 0: colour 0 on even planes
+    const bool rowin = gj >= 0 && gj < ny, rowup = y >= 1 && y < TBW - 1 && gj >= 1 && gj <= ny - 2;
+    const int ylo = blockIdx.y == 0 ? 0 : j0, yhi = j0 + T > ny - 2 ? ny - 1 : j0 + T - 1;
+    const int xlo = blockIdx.x == 0 ? 0 : i0, xhi = i0 + T > nx - 2 ? nx - 1 : i0 + T - 1;
+    const int64_t plane = (int64_t)nx * ny, col = (int64_t)gj * nx + gi;
+    double v[TB_MAXZ][2], r[TB_MAXZ][2];
+    bool up[2], out[2];
+    int own[2], nbx[2];
 #pragma unroll
-        for (int u = 0; u < PER; ++u) {
-            const int q = tid + u * TB_NT;
-            const int hi = q % TBW, hj = (q / TBW) % TBW, k = q / (TBW * TBW);
-            const int gi = ib + hi, gj = jb + hj;
-            const bool in = q < nbox && gi >= 0 && gi < nx && gj >= 0 && gj < ny;
-            va[u] = in ? A[idx3(gi, gj, k, nx, ny)] : 0.0;
-            vr[u] = in ? rhs[idx3(gi, gj, k, nx, ny)] : 0.0;
-        }
+    for (int a = 0; a < 2; ++a) {
+        const int par = a ^ q, x = 2 * c + par, g = gi + par;
+        const bool in = rowin && g >= 0 && g < nx;
+        up[a] = rowup && x >= 1 && x < TBW - 1 && g >= 1 && g <= nx - 2;
+        out[a] = in && gj >= ylo && gj <= yhi && g >= xlo && g <= xhi;
+        own[a] = (y * 2 + par) * HX + c;
+        nbx[a] = !up[a] ? own[a] : par ? y * 2 * HX + c + 1 : (y * 2 + 1) * HX + c - 1;
 #pragma unroll
-        for (int u = 0; u < PER; ++u) {
-            const int q = tid + u * TB_NT;
-            if (q < nbox) {
-                const int hi = q % TBW, hj = (q / TBW) % TBW, k = q / (TBW * TBW);
-                box[tb_at(k, hj, hi)] = va[u];
-                rb[tb_at(k, hj, hi)] = vr[u];
-            }
+        for (int k = 0; k < TB_MAXZ; ++k) {
+            const bool ok = in && k < nz;
+            v[k][a] = ok ? A[k * plane + col + par] : 0.0;
+            r[k][a] = ok ? rhs[k * plane + col + par] : 0.0;
         }
     }
+#pragma unroll
+    for (int k = 0; k < TB_MAXZ; ++k) {
+        lds[k * PLANE + own[0]] = v[k][0];
+        lds[k * PLANE + own[1]] = v[k][1];
+    }
     __syncthreads();
-    constexpr int PER_ROW = (TBW - 2) / 2;   // cells of one colour per box row
-    const int rows = (nz - 2) * (TBW - 2);
+    const int dn = y >= 1 ? TBW : 0, dp = y < TBW - 1 ? TBW : 0;
+    auto half = [&](auto first) {   // column 0 from plane 2 - first, column 1 from the other parity
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+            constexpr int N = TB_MAXZ / 2;
+            const int k0 = (decltype(first)::value ^ a) ? 1 : 2;
+            double pn[N];
+#pragma unroll
+            for (int i = 0; i < N; ++i) {
+                const int k = k0 + 2 * i;
+                pn[i] = 0.0;
+                if (k >= TB_MAXZ - 1) continue;
+                const double *p = lds + k * PLANE;
+                const double off = sx * (v[k][1 - a] + p[nbx[a]]) + sy * (p[own[a] - dn] + p[own[a] + dp]) +
+                                   sz * (v[k - 1][a] + v[k + 1][a]);
+                pn[i] = off - r[k][a];
+            }
+            div_by(pn, denom);
+            if (!up[a]) continue;
+#pragma unroll
+            for (int i = 0; i < N; ++i) {
+                const int k = k0 + 2 * i;
+                if (k >= TB_MAXZ - 1 || (!FULL && k > nz - 2)) continue;
+                const double po = v[k][a];
+                v[k][a] = po + omega * (pn[i] - po);
+                lds[k * PLANE + own[a]] = v[k][a];
+            }
+        }
+    };
+    // a wave's rows (four of them); the last half-sweep needs only the tile's,
+    // each one before it a ring more
+    const int w0 = (threadIdx.x & ~63) / HX, w1 = w0 + 63 / HX;
     for (int s = 0; s < nhalf; ++s) {
-        const int c = (color + s) & 1;
-        for (int q = tid; q < rows * PER_ROW; q += TB_NT) {
-            const int row = q / PER_ROW, r = q % PER_ROW;
-            const int hj = 1 + row % (TBW - 2), k = 1 + row / (TBW - 2);
-            const int gj = jb + hj;
-            const int first = 1 + (((ib + 1 + gj + k) & 1) == c ? 0 : 1);
-            const int hi = first + 2 * r;
-            const int gi = ib + hi;
-            if (gi < 1 || gi > nx - 2 || gj < 1 || gj > ny - 2) continue;
-            const int id = tb_at(k, hj, hi);
-            const double off = sx * (box[tb_at(k, hj, hi - 1)] + box[tb_at(k, hj, hi + 1)]) +
-                               sy * (box[tb_at(k, hj - 1, hi)] + box[tb_at(k, hj + 1, hi)]) +
-                               sz * (box[tb_at(k - 1, hj, hi)] + box[tb_at(k + 1, hj, hi)]);
-            const double pn = (off - rb[id]) / denom;
-            const double po = box[id];
-            box[id] = po + omega * (pn - po);
+        const int ring = nhalf - 1 - s;
+        if (w1 >= halo - ring && w0 <= halo + T - 1 + ring) {
+            if ((color + s) & 1) half(std::integral_constant<int, 1>{});
+            else half(std::integral_constant<int, 0>{});
         }
         __syncthreads();
     }
-    // central columns (and the untouched boundary cells next to them) to B
-    for (int q = tid; q < nz * TBT * TBT; q += TB_NT) {
-        const int ci = q % TBT, cj = (q / TBT) % TBT, k = q / (TBT * TBT);
-        const int gi = i0 + ci, gj = j0 + cj;
-        if (gi > nx - 2 || gj > ny - 2) continue;
-        B[idx3(gi, gj, k, nx, ny)] = box[tb_at(k, cj + TBH, ci + TBH)];
-        if (gi == 1) B[idx3(0, gj, k, nx, ny)] = A[idx3(0, gj, k, nx, ny)];
-        if (gi == nx - 2) B[idx3(nx - 1, gj, k, nx, ny)] = A[idx3(nx - 1, gj, k, nx, ny)];
-        if (gj == 1) B[idx3(gi, 0, k, nx, ny)] = A[idx3(gi, 0, k, nx, ny)];
-        if (gj == ny - 2) B[idx3(gi, ny - 1, k, nx, ny)] = A[idx3(gi, ny - 1, k, nx, ny)];
-        if (gi == 1 && gj == 1) B[idx3(0, 0, k, nx, ny)] = A[idx3(0, 0, k, nx, ny)];
-        if (gi == nx - 2 && gj == 1) B[idx3(nx - 1, 0, k, nx, ny)] = A[idx3(nx - 1, 0, k, nx, ny)];
-        if (gi == 1 && gj == ny - 2) B[idx3(0, ny - 1, k, nx, ny)] = A[idx3(0, ny - 1, k, nx, ny)];
-        if (gi == nx - 2 && gj == ny - 2) B[idx3(nx - 1, ny - 1, k, nx, ny)] = A[idx3(nx - 1, ny - 1, k, nx, ny)];
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+        if (!out[a]) continue;
+#pragma unroll
+        for (int k = 0; k < TB_MAXZ; ++k)
+            if (k < nz) B[k * plane + col + (a ^ q)] = v[k][a];
     }
 }
 
@@ -1581,7 +1683,6 @@ MGSolver::MGSolver(const llgmi_grid &g, const llgmi_mg_config &cfg_in, hipStream
     mg_sanitize(cfg_);
     if (const char *e = std::getenv("LLGMI_MG_GRAPH")) use_graphs_ = std::string(e) != "0";
     if (const char *e = std::getenv("LLGMI_MG_RB_FUSED")) rb_fused_ = std::string(e) != "0";
-    if (const char *e = std::getenv("LLGMI_MG_RBZ")) rbz_ = std::max(1, std::atoi(e));
     try {
         // new_with_operator (:1425-1577)
         const int64_t nx = std::max<int64_t>(g.nx, 1), ny = std::max<int64_t>(g.ny, 1);
@@ -1643,8 +1744,11 @@ MGSolver::MGSolver(const llgmi_grid &g, const llgmi_mg_config &cfg_in, hipStream
             LLGMI_HIP(hipMalloc(&L.d_st, sizeof(DevStencil)));
             LLGMI_HIP(hipMemcpy(L.d_st, &h, sizeof(DevStencil), hipMemcpyHostToDevice));
         }
-        LLGMI_HIP(hipFuncSetAttribute((const void *)k_mg_rb_tb, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      (int)(2 * sizeof(double) * TB_MAXZ * TBW * TBW)));
+        for (const void *k : {(const void *)k_mg_rb_tb<true>, (const void *)k_mg_rb_tb<false>})
+            LLGMI_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                          (int)(sizeof(double) * TB_MAXZ * TBW * TBW)));
+        LLGMI_HIP(hipFuncSetAttribute((const void *)k_mg_rb_sweep2<64, 32>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                      (int)(sizeof(double) * (8 * 64 * 32 + 2 * 64))));
         const size_t n0 = (size_t)px_ * py_ * pz_;
         LLGMI_HIP(hipMalloc((void **)&bc_, sizeof(double) * n0));
         LLGMI_HIP(hipMemsetAsync(bc_, 0, sizeof(double) * n0, stream_));
@@ -1922,34 +2026,26 @@ void MGSolver::smooth(int l, int64_t iters) {
     Level &L = lev_[l];
     if (cfg_.smoother == 1) {
         const double sx = 1.0 / (L.dx * L.dx), sy = 1.0 / (L.dy * L.dy), sz = 1.0 / (L.dz * L.dz);
-        const double denom = 2.0 * (sx + sy + sz);
+        const ExactDiv denom = exact_div(2.0 * (sx + sy + sz));
         const bool coarsest = l == (int)lev_.size() - 1;
-        if (rb_fused_ && l == 0) {
-            // finest level: one fused kernel per sweep
-            ensure_pair(L);
-            const int rbz = std::max(1, std::min(rbz_, L.nz - 2));
-            const dim3 grid((unsigned)((L.nx - 2 + RBX - 1) / RBX), (unsigned)((L.ny - 2 + RBY - 1) / RBY),
-                            (unsigned)((L.nz - 2 + rbz - 1) / rbz));
-            for (int64_t it = 0; it < iters; ++it) {
-                hipLaunchKernelGGL(k_mg_rb_sweep, grid, dim3(RBX * RBY), 0, stream_, L.phi[L.cur],
-                                   L.phi[1 - L.cur], L.rhs, L.nx, L.ny, L.nz, sx, sy, sz, denom, cfg_.sor_omega,
-                                   rbz);
-                LLGMI_LAUNCH_CHECK();
-                L.cur = 1 - L.cur;
-            }
-            return;
-        }
         if (rb_fused_ && coarsest && l > 0 && L.nz <= TB_MAXZ) {
-            // small coarsest level: TBH half-sweeps per launch in LDS
+            // small coarsest level: many half-sweeps per launch in LDS.  The
+            // tile grows by two columns (one half-sweep less per launch) until
+            // every block has a CU of its own.
             ensure_pair(L);
-            const dim3 grid((unsigned)((L.nx - 2 + TBT - 1) / TBT), (unsigned)((L.ny - 2 + TBT - 1) / TBT));
-            const size_t lds = 2 * sizeof(double) * (size_t)L.nz * TBW * TBW;
+            auto blocks = [&](int T) {
+                return (int64_t)((L.nx - 2 + T - 1) / T) * ((L.ny - 2 + T - 1) / T);
+            };
+            int T = 8;
+            while (T < TBW - 8 && blocks(T) > 256) T += 2;
+            const dim3 grid((unsigned)((L.nx - 2 + T - 1) / T), (unsigned)((L.ny - 2 + T - 1) / T));
+            const size_t lds = sizeof(double) * TB_MAXZ * TBW * TBW;
             int64_t left = 2 * iters;
             int color = 0;
             while (left > 0) {
-                const int h = (int)std::min<int64_t>(left, TBH);
-                hipLaunchKernelGGL(k_mg_rb_tb, grid, dim3(TB_NT), lds, stream_, L.phi[L.cur], L.phi[1 - L.cur],
-                                   L.rhs, L.nx, L.ny, L.nz, sx, sy, sz, denom, cfg_.sor_omega, color, h);
+                const int h = (int)std::min<int64_t>(left, (TBW - T) / 2);
+                hipLaunchKernelGGL(L.nz == TB_MAXZ ? k_mg_rb_tb<true> : k_mg_rb_tb<false>, grid, dim3(TB_NT), lds,
+                                   stream_, L.phi[L.cur], L.phi[1 - L.cur], L.rhs, L.nx, L.ny, L.nz, sx, sy, sz, denom, cfg_.sor_omega, color, h, T);
                 LLGMI_LAUNCH_CHECK();
                 L.cur = 1 - L.cur;
                 color = (color + h) & 1;
@@ -1957,7 +2053,26 @@ void MGSolver::smooth(int l, int64_t iters) {
             }
             return;
         }
-        // other levels: the two half-sweep kernels, in place
+        if (rb_fused_ && L.nz >= 3) {
+            // pairs of sweeps; the 64 x 32 box where its blocks fill at least
+            // half the CUs (its halo is re-read and recomputed least), else 32 x 16
+            ensure_pair(L);
+            auto pair_of = [&](auto bxc, auto byc) {
+                constexpr int BX = decltype(bxc)::value, BY = decltype(byc)::value;
+                const dim3 grid((unsigned)((L.nx - 2 + BX - 9) / (BX - 8)), (unsigned)((L.ny - 2 + BY - 9) / (BY - 8)));
+                hipLaunchKernelGGL((k_mg_rb_sweep2<BX, BY>), grid, dim3(BX * BY / 2), sizeof(double) * (8 * BX * BY + 2 * BX),
+                                   stream_, L.phi[L.cur], L.phi[1 - L.cur], L.rhs, L.nx, L.ny, L.nz, sx, sy, sz, denom,
+                                   cfg_.sor_omega);
+                LLGMI_LAUNCH_CHECK();
+                L.cur = 1 - L.cur;
+            };
+            const bool large = (int64_t)((L.nx - 2 + 55) / 56) * ((L.ny - 2 + 23) / 24) >= 128;
+            for (; iters >= 2; iters -= 2) {
+                if (large) pair_of(std::integral_constant<int, 64>{}, std::integral_constant<int, 32>{});
+                else pair_of(std::integral_constant<int, 32>{}, std::integral_constant<int, 16>{});
+            }
+        }
+        // single sweeps: the two half-sweep kernels, in place
         const int64_t n = (int64_t)(L.ny - 2) * (L.nz - 2) * ((L.nx - 1) / 2);
         for (int64_t it = 0; it < iters; ++it)
             for (int color = 0; color < 2; ++color) {

@@ -111,7 +111,6 @@ private:
     std::map<std::string, Graph> graphs_;
     bool use_graphs_ = true;   // LLGMI_MG_GRAPH=0: launch the V-cycle kernels directly
     bool rb_fused_ = true;     // LLGMI_MG_RB_FUSED=0: two half-sweep launches per sweep
-    int rbz_ = 1 << 20;        // LLGMI_MG_RBZ: planes per z-chunk of the fused finest sweep
 };
 
 // Hybrid MG correction (DeltaKernel2D::add_correction, demag_poisson_mg.rs:410-583):

@@ -61,6 +61,30 @@ def test_mg_fp64_matches_oracle_with_warm_start(gpu_lib, op, bc):
             assert st["tree_rebuilt"] == (solve != 1)
 
 
+# Smoothers on the edges of their tiles, a few cycles without a tolerance, zero
+# boundary: two-sweep boxes of 32 x 16 (24 x 8 columns) with one, full and
+# remainder tiles, odd sweep counts (the last one in place), coarsest levels of
+# nine and fewer planes and of several tiles, a flat box and one that does not
+# coarsen in the plane; 640 x 600 takes the 64 x 32 boxes.
+@pytest.mark.parametrize("nx,ny,nvac,pre,post,cycles", [
+    (7, 5, 3, 2, 2, 3), (26, 10, 4, 2, 1, 3), (27, 41, 8, 3, 2, 3), (50, 34, 16, 1, 4, 3), (75, 12, 16, 2, 3, 3),
+    (131, 90, 5, 2, 2, 2), (640, 600, 2, 2, 2, 1)])
+@pytest.mark.parametrize("op", ["rb7_inject_rd", "iso27_tri_galerkin"])
+def test_mg_smoother_tile_edges(gpu_lib, nx, ny, nvac, pre, post, cycles, op):
+    from oracle import oracle as O
+    L = gpu_lib
+    cell = (4e-9, 3e-9, 2e-9)
+    lc, oc = _pair(L, O, pad_xy=2, n_vac_z=nvac, bc=0, pre_smooth=pre, post_smooth=post, warm_start=0, tol_rel=None,
+                   tol_abs=None, v_cycles=cycles, sor_omega=1.2, **OPS[op])
+    m = _rand_m(nx * ny, nx + ny, (0, nx * ny // 2))
+    want = np.zeros_like(m)
+    O.MG(O.Grid(nx, ny, *cell), oc).add_field(m, want, 8e5)
+    ctx = L.Context(L.Grid2D(nx, ny, *cell), precision=L.F64)
+    ctx.set_mg_config(lc)
+    got = ctx.compute_demag_field_poisson_mg(m, L.Material(ms=8e5, demag=True))
+    assert rel_err(got, want) <= 1e-12
+
+
 @pytest.mark.parametrize("op", ["rb7_inject_rd", "iso27_tri_galerkin"])
 def test_mg_fp32_context_close_to_oracle(gpu_lib, op):
     from oracle import oracle as O
