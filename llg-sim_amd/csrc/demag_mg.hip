@@ -48,9 +48,10 @@ constexpr int kNT = 256;
 
 struct DevStencil {
     double center, diag;
-    int n, pad_;
+    int n, near;              // near: no offset beyond one cell, lin valid
     double c[kMaxSt];
     int off[kMaxSt][3];
+    int64_t lin[kMaxSt];      // off as index distances in the level's box
 };
 
 struct TNode {            // octree node in pre-order; leaf iff count > 0
@@ -130,6 +131,24 @@ __device__ __forceinline__ double offdiag(const double *__restrict__ phi, int nx
         const int jj = clampi(j + st->off[q][1], 0, ny - 1);
         const int kk = clampi(k + st->off[q][2], 0, nz - 1);
         sum += st->c[q] * phi[idx3(ii, jj, kk, nx, ny)];
+    }
+    return sum;
+}
+
+// The same at an interior cell id: the clamp never acts on offsets of one cell,
+// so the sum is over fixed index distances (uniform over the wave), in the
+// stencil's order.
+__device__ __forceinline__ double offdiag_in(const double *__restrict__ phi, int64_t id, int nx, int ny, int nz,
+                                             int i, int j, int k, const DevStencil *__restrict__ st) {
+    if (!st->near) return offdiag(phi, nx, ny, nz, i, j, k, st);
+    const double *p = phi + id;
+    double sum = 0.0;
+    const int n = st->n;
+    if (n == 26) {
+#pragma unroll
+        for (int q = 0; q < 26; ++q) sum += st->c[q] * p[st->lin[q]];
+    } else {
+        for (int q = 0; q < n; ++q) sum += st->c[q] * p[st->lin[q]];
     }
     return sum;
 }
@@ -511,26 +530,118 @@ __global__ void __launch_bounds__(TB_NT) k_mg_rb_tb(const double *__restrict__ A
     }
 }
 
+// Cell of a thread of the grids below (blocks of 64 x 4 cells of one plane, one
+// plane per blockIdx.z): no division per cell.
+constexpr int kBX = 64, kBY = 4;
+__device__ __forceinline__ int cell_i() { return (int)(blockIdx.x * kBX + threadIdx.x); }
+__device__ __forceinline__ int cell_j() { return (int)(blockIdx.y * kBY + threadIdx.y); }
+inline dim3 cell_grid(int nx, int ny, int nz) {
+    return dim3((unsigned)((nx + kBX - 1) / kBX), (unsigned)((ny + kBY - 1) / kBY), (unsigned)nz);
+}
+
 // One sweep of smooth_weighted_jacobi from src into dst; boundary cells of dst
 // take the Dirichlet values (bc, or 0 when bc is null).
-__global__ void __launch_bounds__(kNT) k_mg_wj(const double *__restrict__ src, double *__restrict__ dst,
-                                               const double *__restrict__ rhs, const double *__restrict__ bc,
-                                               const DevStencil *__restrict__ st, double omega, int nx,
-                                               int ny, int nz) {
-    const int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (id >= (int64_t)nx * ny * nz) return;
-    const int i = (int)(id % nx);
-    const int64_t r = id / nx;
-    const int j = (int)(r % ny);
-    const int k = (int)(r / ny);
+__global__ void __launch_bounds__(kBX *kBY) k_mg_wj(const double *__restrict__ src, double *__restrict__ dst,
+                                                    const double *__restrict__ rhs, const double *__restrict__ bc,
+                                                    const DevStencil *__restrict__ st, ExactDiv diag, double omega,
+                                                    int nx, int ny, int nz) {
+    const int i = cell_i(), j = cell_j(), k = (int)blockIdx.z;
+    if (i >= nx || j >= ny) return;
+    const int64_t id = idx3(i, j, k, nx, ny);
     if (i == 0 || i == nx - 1 || j == 0 || j == ny - 1 || k == 0 || k == nz - 1) {
         dst[id] = bc ? bc[id] : 0.0;
         return;
     }
-    const double off = offdiag(src, nx, ny, nz, i, j, k, st);
+    const double off = offdiag_in(src, id, nx, ny, nz, i, j, k, st);
     const double s = src[id];
-    const double gs = fabs(st->diag) > 1e-30 ? (off - rhs[id]) / st->diag : s;
-    dst[id] = (1.0 - omega) * s + omega * gs;
+    double gs[1] = {off - rhs[id]};
+    if (fabs(diag.d) > 1e-30) div_by(gs, diag);
+    else gs[0] = s;
+    dst[id] = (1.0 - omega) * s + omega * gs[0];
+}
+
+// `nsweep` weighted-Jacobi sweeps in one launch, for small levels of at most
+// TB_MAXZ planes with zero boundary values and a stencil of radius one whose
+// terms come in lexicographic (x, y, z) order, the order of the Galerkin coarse
+// operators (coefficients c[(dx+1) 9 + (dy+1) 3 + dz+1], centre unused).  A block
+// holds a WJW x WJW x nz box, the central T x T columns of which are exact after
+// (WJW - T) / 2 sweeps; a thread owns one column.  The nine columns around it
+// are read from LDS once each and every value serves the three cells above,
+// beside and below it (81 reads per sweep and thread against 182): for each cell
+// the terms still arrive in the stencil's order.
+// The 80 sweeps of the coarsest level of a 200 x 160 film (53 x 43 x 9) took 80
+// launches of 7 to 9 us, nearly all of it launch and drain; a launch lasts as
+// long as one block, so the host takes the narrowest tile whose blocks still
+// find a CU each.
+// Measured there: 80 sweeps in 14 launches of 11.6 us (163 us) against 750 us.
+struct WjCoef {
+    double c[27];
+};
+constexpr int WJW = 16, WJ_PAD = WJW + 1;
+__global__ void __launch_bounds__(WJW *WJW) k_mg_wj_tb(const double *__restrict__ A, double *__restrict__ B,
+                                                       const double *__restrict__ rhs, int nx, int ny, int nz,
+                                                       WjCoef st, ExactDiv diag, double omega, int nsweep, int T) {
+    constexpr int PLANE = WJW * WJW;
+    __shared__ double box[TB_MAXZ * PLANE + 2 * WJ_PAD];
+    double *lds = box + WJ_PAD;   // edge threads read (and drop) past the planes
+    const int x = threadIdx.x % WJW, y = threadIdx.x / WJW, halo = (WJW - T) / 2;
+    const int i0 = 1 + (int)blockIdx.x * T, j0 = 1 + (int)blockIdx.y * T;
+    const int gi = i0 - halo + x, gj = j0 - halo + y;
+    const bool in = gi >= 0 && gi < nx && gj >= 0 && gj < ny;
+    const bool up = x >= 1 && x < WJW - 1 && y >= 1 && y < WJW - 1 && gi >= 1 && gi <= nx - 2 && gj >= 1 && gj <= ny - 2;
+    const int ylo = blockIdx.y == 0 ? 0 : j0, yhi = j0 + T > ny - 2 ? ny - 1 : j0 + T - 1;
+    const int xlo = blockIdx.x == 0 ? 0 : i0, xhi = i0 + T > nx - 2 ? nx - 1 : i0 + T - 1;
+    const int64_t plane = (int64_t)nx * ny, col = (int64_t)gj * nx + gi;
+    double v[TB_MAXZ], r[TB_MAXZ];
+#pragma unroll
+    for (int k = 0; k < TB_MAXZ; ++k) {
+        v[k] = in && k < nz ? A[k * plane + col] : 0.0;
+        r[k] = in && k < nz ? rhs[k * plane + col] : 0.0;
+    }
+#pragma unroll
+    for (int k = 0; k < TB_MAXZ; ++k) lds[k * PLANE + (int)threadIdx.x] = v[k];
+    __syncthreads();
+    const int w0 = (threadIdx.x & ~63) / WJW, w1 = w0 + 63 / WJW;   // the wave's rows
+    for (int s = 0; s < nsweep; ++s) {
+        const int ring = nsweep - 1 - s;
+        const bool need = w1 >= halo - ring && w0 <= halo + T - 1 + ring;
+        double g[TB_MAXZ - 2];
+        if (need) {
+#pragma unroll
+            for (int k = 0; k < TB_MAXZ - 2; ++k) g[k] = 0.0;
+#pragma unroll
+            for (int n = 0; n < 9; ++n) {
+                const int dx = n / 3 - 1, dy = n % 3 - 1;
+                double c[TB_MAXZ];
+#pragma unroll
+                for (int k = 0; k < TB_MAXZ; ++k) c[k] = n == 4 ? v[k] : lds[k * PLANE + (int)threadIdx.x + dy * WJW + dx];
+#pragma unroll
+                for (int k = 1; k < TB_MAXZ - 1; ++k)
+#pragma unroll
+                    for (int dz = -1; dz <= 1; ++dz)
+                        if (n != 4 || dz != 0) g[k - 1] += st.c[n * 3 + dz + 1] * c[k + dz];
+            }
+#pragma unroll
+            for (int k = 0; k < TB_MAXZ - 2; ++k) g[k] -= r[k + 1];
+            div_by(g, diag);
+        }
+        __syncthreads();   // the sweep's reads are done
+        if (need && up) {
+#pragma unroll
+            for (int k = 1; k < TB_MAXZ - 1; ++k) {
+                if (k > nz - 2) continue;
+                v[k] = (1.0 - omega) * v[k] + omega * g[k - 1];
+                lds[k * PLANE + (int)threadIdx.x] = v[k];
+            }
+        }
+        __syncthreads();
+    }
+    if (in && gj >= ylo && gj <= yhi && gi >= xlo && gi <= xhi) {
+        const bool edge = gi == 0 || gi == nx - 1 || gj == 0 || gj == ny - 1;
+#pragma unroll
+        for (int k = 0; k < TB_MAXZ; ++k)
+            if (k < nz) B[k * plane + col] = edge || k == 0 || k == nz - 1 ? 0.0 : v[k];
+    }
 }
 
 __device__ __forceinline__ double block_max(double v) {
@@ -552,18 +663,19 @@ __global__ void __launch_bounds__(kNT) k_mg_resid_max(const double *__restrict__
                                                       const double *__restrict__ rhs,
                                                       const DevStencil *__restrict__ st, int nx, int ny,
                                                       int nz, int seven, double *__restrict__ partial) {
-    const int64_t n = (int64_t)(nx - 2) * (ny - 2) * (nz - 2);
+    // a wave takes whole rows, so the row's position is uniform
     const int64_t plane = (int64_t)nx * ny;
+    const int rows = (ny - 2) * (nz - 2), nw = (int)gridDim.x * (kNT / 64), lane = threadIdx.x & 63;
     double mx = 0.0;
-    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (int64_t)gridDim.x * blockDim.x) {
-        const int i = 1 + (int)(t % (nx - 2));
-        const int64_t r = t / (nx - 2);
-        const int j = 1 + (int)(r % (ny - 2));
-        const int k = 1 + (int)(r / (ny - 2));
-        const int64_t id = idx3(i, j, k, nx, ny);
-        const double a = st->center * phi[id] +
-                         (seven ? offdiag7(phi, id, nx, plane, st) : offdiag(phi, nx, ny, nz, i, j, k, st));
-        mx = fmax(mx, fabs(rhs[id] - a));
+    for (int row = __builtin_amdgcn_readfirstlane((int)blockIdx.x * (kNT / 64) + (int)(threadIdx.x >> 6)); row < rows;
+         row += nw) {
+        const int k = 1 + row / (ny - 2), j = 1 + row % (ny - 2);
+        for (int i = 1 + lane; i <= nx - 2; i += 64) {
+            const int64_t id = idx3(i, j, k, nx, ny);
+            const double a = st->center * phi[id] + (seven ? offdiag7(phi, id, nx, plane, st)
+                                                           : offdiag_in(phi, id, nx, ny, nz, i, j, k, st));
+            mx = fmax(mx, fabs(rhs[id] - a));
+        }
     }
     mx = block_max(mx);
     if (threadIdx.x == 0) partial[blockIdx.x] = mx;
@@ -571,20 +683,15 @@ __global__ void __launch_bounds__(kNT) k_mg_resid_max(const double *__restrict__
 
 // Residual + restrict_residual: coarse rhs = mean over the fine block of
 // r = rhs - A phi; coarse phi = 0 (interior; the coarse boundary stays 0).
-__global__ void __launch_bounds__(kNT) k_mg_resid_restrict(const double *__restrict__ phi,
+__global__ void __launch_bounds__(kBX *kBY) k_mg_resid_restrict(const double *__restrict__ phi,
                                                            const double *__restrict__ rhs,
                                                            const DevStencil *__restrict__ st, int fnx,
                                                            int fny, int fnz, double *__restrict__ crhs,
                                                            double *__restrict__ cphi, int cnx, int cny,
                                                            int cnz, int rx, int ry, int rz, double w,
                                                            int seven) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t n = (int64_t)(cnx - 2) * (cny - 2) * (cnz - 2);
-    if (t >= n) return;
-    const int ic = 1 + (int)(t % (cnx - 2));
-    const int64_t r = t / (cnx - 2);
-    const int jc = 1 + (int)(r % (cny - 2));
-    const int kc = 1 + (int)(r / (cny - 2));
+    const int ic = 1 + cell_i(), jc = 1 + cell_j(), kc = 1 + (int)blockIdx.z;
+    if (ic > cnx - 2 || jc > cny - 2) return;
     double sum = 0.0;
     for (int dk = 0; dk < rz; ++dk)
         for (int dj = 0; dj < ry; ++dj)
@@ -593,7 +700,7 @@ __global__ void __launch_bounds__(kNT) k_mg_resid_restrict(const double *__restr
                 const int64_t id = idx3(i, j, k, fnx, fny);
                 const double a = st->center * phi[id] +
                                  (seven ? offdiag7(phi, id, fnx, (int64_t)fnx * fny, st)
-                                        : offdiag(phi, fnx, fny, fnz, i, j, k, st));
+                                        : offdiag_in(phi, id, fnx, fny, fnz, i, j, k, st));
                 sum += rhs[id] - a;
             }
     const int64_t cid = idx3(ic, jc, kc, cnx, cny);
@@ -624,16 +731,11 @@ __device__ __forceinline__ void interp_1d(int ic, int ri, int nc, int r, int &i0
 }
 
 // prolongate_add (mg_kernels.rs:377-439), one thread per fine interior cell
-__global__ void __launch_bounds__(kNT) k_mg_prolong(const double *__restrict__ c, int cnx, int cny, int cnz,
+__global__ void __launch_bounds__(kBX *kBY) k_mg_prolong(const double *__restrict__ c, int cnx, int cny, int cnz,
                                                     double *__restrict__ f, int fnx, int fny, int fnz,
                                                     int trilinear) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t n = (int64_t)(fnx - 2) * (fny - 2) * (fnz - 2);
-    if (t >= n) return;
-    const int i = 1 + (int)(t % (fnx - 2));
-    const int64_t r = t / (fnx - 2);
-    const int j = 1 + (int)(r % (fny - 2));
-    const int k = 1 + (int)(r / (fny - 2));
+    const int i = 1 + cell_i(), j = 1 + cell_j(), k = 1 + (int)blockIdx.z;
+    if (i > fnx - 2 || j > fny - 2) return;
     const int rx = fnx / cnx, ry = fny / cny, rz = fnz / cnz;
     const int64_t id = idx3(i, j, k, fnx, fny);
     if (trilinear) {
@@ -1737,9 +1839,14 @@ MGSolver::MGSolver(const llgmi_grid &g, const llgmi_mg_config &cfg_in, hipStream
             h.center = L.st.center;
             h.diag = L.st.diag;
             h.n = (int)L.st.coeffs.size();
+            h.near = 1;
             for (int q = 0; q < h.n; ++q) {
                 h.c[q] = L.st.coeffs[q];
-                for (int a = 0; a < 3; ++a) h.off[q][a] = L.st.offs[q][a];
+                for (int a = 0; a < 3; ++a) {
+                    h.off[q][a] = L.st.offs[q][a];
+                    if (std::abs(h.off[q][a]) > 1) h.near = 0;
+                }
+                h.lin[q] = ((int64_t)h.off[q][2] * L.ny + h.off[q][1]) * L.nx + h.off[q][0];
             }
             LLGMI_HIP(hipMalloc(&L.d_st, sizeof(DevStencil)));
             LLGMI_HIP(hipMemcpy(L.d_st, &h, sizeof(DevStencil), hipMemcpyHostToDevice));
@@ -2022,6 +2129,24 @@ void MGSolver::ensure_pair(Level &L) {
     LLGMI_HIP(hipMemsetAsync(L.phi[1], 0, sizeof(double) * n, stream_));
 }
 
+// Whether every offset is within one cell and the terms come in strictly
+// ascending (x, y, z) order without the centre; then their coefficients by place.
+// A place without a term gets 0, whose product leaves a finite sum as it is.
+static bool lexicographic(const MGStencil &st, WjCoef &co) {
+    std::fill(co.c, co.c + 27, 0.0);
+    int last = -1;
+    for (size_t q = 0; q < st.offs.size(); ++q) {
+        const auto &o = st.offs[q];
+        for (int a = 0; a < 3; ++a)
+            if (o[a] < -1 || o[a] > 1) return false;
+        const int at = (o[0] + 1) * 9 + (o[1] + 1) * 3 + o[2] + 1;
+        if (at <= last || at == 13) return false;
+        last = at;
+        co.c[at] = st.coeffs[q];
+    }
+    return true;
+}
+
 void MGSolver::smooth(int l, int64_t iters) {
     Level &L = lev_[l];
     if (cfg_.smoother == 1) {
@@ -2083,10 +2208,28 @@ void MGSolver::smooth(int l, int64_t iters) {
         return;
     }
     ensure_pair(L);
-    const int64_t n = (int64_t)L.nx * L.ny * L.nz;
+    const ExactDiv diag = exact_div(L.st.diag);
+    WjCoef co;
+    if (l > 0 && l == (int)lev_.size() - 1 && L.nz <= TB_MAXZ && std::fabs(L.st.diag) > 1e-30 && lexicographic(L.st, co)) {
+        // several sweeps per launch; the tile grows until every block has a CU
+        auto blocks = [&](int T) { return (int64_t)((L.nx - 2 + T - 1) / T) * ((L.ny - 2 + T - 1) / T); };
+        int T = 4;
+        while (T < WJW - 4 && blocks(T) > 256) T += 2;
+        const dim3 grid((unsigned)((L.nx - 2 + T - 1) / T), (unsigned)((L.ny - 2 + T - 1) / T));
+        for (int64_t left = iters; left > 0;) {
+            const int h = (int)std::min<int64_t>(left, (WJW - T) / 2);
+            hipLaunchKernelGGL(k_mg_wj_tb, grid, dim3(WJW * WJW), 0, stream_, L.phi[L.cur], L.phi[1 - L.cur], L.rhs,
+                               L.nx, L.ny, L.nz, co, diag, cfg_.omega, h, T);
+            LLGMI_LAUNCH_CHECK();
+            L.cur = 1 - L.cur;
+            left -= h;
+        }
+        return;
+    }
     for (int64_t it = 0; it < iters; ++it) {
-        hipLaunchKernelGGL(k_mg_wj, dim3(nblocks(n)), dim3(kNT), 0, stream_, L.phi[L.cur], L.phi[1 - L.cur], L.rhs,
-                           l == 0 ? bc_ : nullptr, (const DevStencil *)L.d_st, cfg_.omega, L.nx, L.ny, L.nz);
+        hipLaunchKernelGGL(k_mg_wj, cell_grid(L.nx, L.ny, L.nz), dim3(kBX, kBY), 0, stream_, L.phi[L.cur],
+                           L.phi[1 - L.cur], L.rhs, l == 0 ? bc_ : nullptr, (const DevStencil *)L.d_st, diag, cfg_.omega,
+                           L.nx, L.ny, L.nz);
         LLGMI_LAUNCH_CHECK();
         L.cur = 1 - L.cur;
     }
@@ -2101,14 +2244,12 @@ void MGSolver::v_cycle(int l) {
     smooth(l, cfg_.pre_smooth);
     Level &F = lev_[l], &C = lev_[l + 1];
     const int rx = F.nx / C.nx, ry = F.ny / C.ny, rz = F.nz / C.nz;
-    const int64_t nc = (int64_t)(C.nx - 2) * (C.ny - 2) * (C.nz - 2);
-    hipLaunchKernelGGL(k_mg_resid_restrict, dim3(nblocks(nc)), dim3(kNT), 0, stream_, F.phi[F.cur], F.rhs,
+    if (C.nx > 2 && C.ny > 2 && C.nz > 2) hipLaunchKernelGGL(k_mg_resid_restrict, cell_grid(C.nx - 2, C.ny - 2, C.nz - 2), dim3(kBX, kBY), 0, stream_, F.phi[F.cur], F.rhs,
                        (const DevStencil *)F.d_st, F.nx, F.ny, F.nz, C.rhs, C.phi[C.cur], C.nx, C.ny, C.nz, rx, ry,
                        rz, 1.0 / (double)(rx * ry * rz), F.seven ? 1 : 0);
     LLGMI_LAUNCH_CHECK();
     v_cycle(l + 1);
-    const int64_t nf = (int64_t)(F.nx - 2) * (F.ny - 2) * (F.nz - 2);
-    hipLaunchKernelGGL(k_mg_prolong, dim3(nblocks(nf)), dim3(kNT), 0, stream_, C.phi[C.cur], C.nx, C.ny, C.nz,
+    hipLaunchKernelGGL(k_mg_prolong, cell_grid(F.nx - 2, F.ny - 2, F.nz - 2), dim3(kBX, kBY), 0, stream_, C.phi[C.cur], C.nx, C.ny, C.nz,
                        F.phi[F.cur], F.nx, F.ny, F.nz, cfg_.prolong == 1 ? 1 : 0);
     LLGMI_LAUNCH_CHECK();
     smooth(l, cfg_.post_smooth);
