@@ -132,7 +132,9 @@ __device__ __forceinline__ uint4 relu_mask(uint4 v, uint4 m) {
 // Requires cin % 16 == 0, cout % (16*NT) == 0; H, W even for pool and CAT.
 // Measured against the tap-by-tap tile kernel with separate pooling, upsampling,
 // concatenation, ReLU-gradient and loss passes: forward at 528 x 528 467 -> 365
-// us, training step at batch 8 8.10 -> 5.84 ms.
+// us, training step at batch 8 8.10 -> 5.84 ms; with the loss's targets through
+// LDS, three blocks per CU for the 16-wide tiles and even runs of tiles 333 us and
+// 5.59 ms.
 constexpr int kKC = 32, kKRow = kKC + 8;   // channel chunk; LDS row, padded against bank conflicts
 template <int TH, int TW, int NT>
 struct ConvShape {
@@ -140,8 +142,11 @@ struct ConvShape {
     static constexpr int kXin = NPX * kKRow, kOut = NOUT * (CO + 8), kReg = kXin > kOut ? kXin : kOut;
     static constexpr size_t LDS = sizeof(uint16_t) * (size_t)(kReg + 9 * CO * kKRow);
 };
+// blocks per CU a tile's registers and LDS allow
+template <int TW, int NT>
+constexpr int conv_blocks_per_cu() { return TW == 1 && NT < 3 ? 3 : 2; }
 template <int TH, int TW, int NT, int EPI, bool RELU>
-__global__ __launch_bounds__(256, 2) void k_conv3x3(ConvSrc src, int cin, const uint16_t *__restrict__ w,
+__global__ __launch_bounds__(256, (conv_blocks_per_cu<TW, NT>())) void k_conv3x3(ConvSrc src, int cin, const uint16_t *__restrict__ w,
                                                     const float *__restrict__ bias, ConvEpi ep, int cout, int B,
                                                     int H, int W) {
     using S = ConvShape<TH, TW, NT>;
@@ -269,6 +274,21 @@ __global__ __launch_bounds__(256, 2) void k_conv3x3(ConvSrc src, int cin, const 
             continue;
         }
         __syncthreads();   // every wave's reads of xin are done
+        if constexpr (EPI == EPI_MSE) {
+            // the tile's targets into the places their gradients will take, in
+            // 16-byte pieces (read in the products' layout, two bytes a lane, they
+            // took longer than the convolution)
+            const int tid = opaque(threadIdx.x);
+            for (int e = tid; e < TH * 16 * TW * (CO / 8); e += 256) {
+                const int px = e / (CO / 8), c = (e % (CO / 8)) * 8;
+                const int yy = y0 + px / (16 * TW), xx = x0 + px % (16 * TW);
+                uint4 tv{0u, 0u, 0u, 0u};
+                if (yy < H && xx < W)
+                    tv = *reinterpret_cast<const uint4 *>(ep.tgt + ((int64_t)(b * H + yy) * W + xx) * cout + co_base + c);
+                *reinterpret_cast<uint4 *>(xin + px * OROW + c) = tv;
+            }
+            __syncthreads();
+        }
         if (cat_up) {
             if constexpr (EPI == EPI_CAT) {
 #pragma unroll
@@ -298,18 +318,18 @@ __global__ __launch_bounds__(256, 2) void k_conv3x3(ConvSrc src, int cin, const 
                         for (int q = 0; q < 4; ++q) {
                             float v = acc[r][h][nt][q] + bv;
                             if (RELU) v = fmaxf(v, 0.f);
+                            uint16_t &at = xin[((wave * RW + r) * 16 * TW + h * 16 + g * 4 + q) * OROW + nt * 16 + li];
                             if constexpr (EPI == EPI_MSE) {
                                 const int yy = y0 + wave * RW + r, xx = x0 + h * 16 + g * 4 + q;
                                 float gr = 0.f;
                                 if (co < ep.cv && xx < ep.wv && yy < ep.hv) {
-                                    const double d =
-                                        (double)v - (double)bf2f(ep.tgt[((int64_t)(b * H + yy) * W + xx) * cout + co]);
+                                    const double d = (double)v - (double)bf2f(at);
                                     lsum += d * d;
                                     gr = (float)(2.0 * d * ep.inv_count);
                                 }
                                 v = gr;
                             }
-                            xin[((wave * RW + r) * 16 * TW + h * 16 + g * 4 + q) * OROW + nt * 16 + li] = f2bf(v);
+                            at = f2bf(v);
                         }
                     }
         }
@@ -565,18 +585,27 @@ __global__ void k_adam(float *__restrict__ p, const float *__restrict__ g, float
     }
 }
 
-// bf16 weights for the forward product (same layout) and for the data
-// gradient: wb[tap'][ci][co] = w[8 - tap'][co][ci]
-__global__ void k_w_cast(const float *__restrict__ w, int cout, int cin, uint16_t *__restrict__ wf,
-                         uint16_t *__restrict__ wb) {
-    const int64_t n = (int64_t)9 * cout * cin;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const int ci = (int)(i % cin);
-        const int co = (int)((i / cin) % cout);
-        const int tap = (int)(i / ((int64_t)cin * cout));
+// bf16 weights of every convolution (blockIdx.y) for the forward product (same
+// layout) and for the data gradient: wb[tap'][ci][co] = w[8 - tap'][co][ci].  One
+// launch: a layer's cast is shorter than a launch.
+constexpr int kConvs = 4 * kLevels - 1;
+struct CastLayer {
+    int64_t w_off;
+    int cout, cin;
+    uint16_t *wf, *wb;
+};
+struct CastLayers {
+    CastLayer l[kConvs];
+};
+__global__ void k_w_cast(const float *__restrict__ p, CastLayers layers) {
+    const CastLayer L = layers.l[blockIdx.y];
+    const float *w = p + L.w_off;
+    const int n = 9 * L.cout * L.cin;
+    for (int i = (int)(blockIdx.x * blockDim.x + threadIdx.x); i < n; i += (int)(gridDim.x * blockDim.x)) {
+        const int ci = i % L.cin, co = (i / L.cin) % L.cout, tap = i / (L.cin * L.cout);
         const uint16_t h = f2bf(w[i]);
-        wf[i] = h;
-        wb[((int64_t)(8 - tap) * cin + ci) * cout + co] = h;
+        L.wf[i] = h;
+        L.wb[((8 - tap) * L.cin + ci) * L.cout + co] = h;
     }
 }
 
@@ -793,11 +822,13 @@ struct UNet {
         LLGMI_HIP(hipStreamSynchronize(stream));
     }
     void cast_weights() {
-        for (auto &cv : conv) {
-            const int64_t n = (int64_t)9 * cv.cin * cv.cout;
-            hipLaunchKernelGGL(k_w_cast, dim3(grid_of(n)), dim3(kNT), 0, stream, d_p + cv.w_off, cv.cout, cv.cin,
-                               cv.wf, cv.wb);
+        if (conv.size() != (size_t)kConvs) throw Error(LLGMI_ERR_INVALID, "internal: number of convolutions");
+        CastLayers layers;
+        for (int k = 0; k < kConvs; ++k) {
+            const UNetConv &cv = conv[(size_t)k];
+            layers.l[k] = CastLayer{cv.w_off, cv.cout, cv.cin, cv.wf, cv.wb};
         }
+        hipLaunchKernelGGL(k_w_cast, dim3(128, kConvs), dim3(kNT), 0, stream, d_p, layers);
         LLGMI_LAUNCH_CHECK();
     }
 
@@ -859,8 +890,11 @@ struct UNet {
             }
         }
         const int ntile = ((wl(l) + 16 * TW - 1) / (16 * TW)) * ((hl(l) + TH - 1) / TH) * B, groups = co / (16 * NT);
-        // one-chunk layers run several tiles per block (weights stay in LDS)
-        const int nb = cin <= kKC ? std::min(ntile, std::max(1, 1024 / groups)) : ntile;
+        // one-chunk layers run several tiles per block (weights stay in LDS): as
+        // many as leave one round of resident blocks, the same number each
+        const int64_t slots = 256 * conv_blocks_per_cu<TW, NT>();
+        const int per = cin <= kKC ? (int)(((int64_t)ntile * groups + slots - 1) / slots) : 1;
+        const int nb = (ntile + per - 1) / per;
         hipLaunchKernelGGL(kern, dim3((unsigned)nb, (unsigned)groups), dim3(256), lds, stream, src, cin, w, bias, ep, co,
                            B, hl(l), wl(l));
         LLGMI_LAUNCH_CHECK();
@@ -914,7 +948,7 @@ struct UNet {
     const UNetConv &enc(int l, int k) const { return conv[(size_t)(2 * l + k)]; }
     const UNetConv &dec(int l, int k) const { return conv[(size_t)(2 * kLevels + 2 * (kLevels - 2 - l) + k)]; }
     const UNetConv &head() const { return conv.back(); }
-    static int level_of(int k) { return k < 2 * kLevels ? k / 2 : k == 4 * kLevels - 2 ? 0 : kLevels - 2 - (k - 2 * kLevels) / 2; }
+    static int level_of(int k) { return k < 2 * kLevels ? k / 2 : k == kConvs - 1 ? 0 : kLevels - 2 - (k - 2 * kLevels) / 2; }
 
     // decoder l's input: the upsampled level below and enc_l's output
     ConvSrc cat(int l) const { return {l == kLevels - 2 ? eb[l + 1] : db[l + 1], c(l + 1), eb[l], c(l)}; }
