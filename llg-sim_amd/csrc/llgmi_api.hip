@@ -502,7 +502,7 @@ struct Engine : EngineBase {
         const bool demag = mask == LLGMI_MASK_FULL && mat.demag;
         LocalArgs<T> a = local_args(p, mat, mask, kout != nullptr, relax);
         if (nxt) {
-            if (!kout || relax || nxt->nk < 1 || nxt->nk > 5 || nxt->k[nxt->nk - 1] != kout)
+            if (!kout || nxt->nk < 1 || nxt->nk > 5 || nxt->k[nxt->nk - 1] != kout)
                 throw Error(LLGMI_ERR_INVALID, "fused RK stage: the last slope must be this evaluation's torque");
             a.st_out = nxt_out;
             a.st_m = nxt_m;
@@ -974,6 +974,7 @@ struct Engine : EngineBase {
         alloc(d_r23b4, 3 * n);
         alloc(d_r23m4, 3 * n);
         alloc(d_stage, 3 * n);
+        alloc(d_stage2, 3 * n);
         alloc(d_b, 3 * n);
         ensure_red();
     }
@@ -1011,10 +1012,27 @@ struct Engine : EngineBase {
             launch_rk_stage<T>(m, sa, out, n, stream);
         };
         stage({{K[1], A21}}, d_stage);
-        field(d_stage, d_b, p, mat, mask, nullptr, K[2], true);
-        stage({{K[2], A32}}, d_stage);
-        field(d_stage, d_b, p, mat, mask, nullptr, K[3], true);
-        stage({{K[1], B1}, {K[2], B2}, {K[3], B3}}, d_r23m4);
+        if (rk45_fuse_enabled()) {
+            // as in rk45_stages: the next state is formed in the field
+            // evaluation's epilogue, and a stage's field is not stored
+            StageArgs<T> s3{}, s4{};
+            s3.nk = 1;
+            s3.k[0] = K[2];
+            s3.c[0] = T(dt0 * A32);
+            field(d_stage, nullptr, p, mat, mask, nullptr, K[2], true, &s3, m, d_stage2);
+            s4.nk = 3;
+            const double w[3] = {B1, B2, B3};
+            for (int q = 0; q < 3; ++q) {
+                s4.k[q] = K[q + 1];
+                s4.c[q] = T(dt0 * w[q]);
+            }
+            field(d_stage2, nullptr, p, mat, mask, nullptr, K[3], true, &s4, m, d_r23m4);
+        } else {
+            field(d_stage, d_b, p, mat, mask, nullptr, K[2], true);
+            stage({{K[2], A32}}, d_stage);
+            field(d_stage, d_b, p, mat, mask, nullptr, K[3], true);
+            stage({{K[1], B1}, {K[2], B2}, {K[3], B3}}, d_r23m4);
+        }
         field(d_r23m4, d_r23b4, p, mat, mask, nullptr, K[4], true);
         {
             Rk23ErrCoef c{{dt0 * B1, dt0 * B2, dt0 * B3}, {dt0 * BH1, dt0 * BH2, dt0 * BH3, dt0 * BH4}};

@@ -244,3 +244,45 @@ def test_relax_argument_errors(gpu_lib):
     with pytest.raises(L.LlgmiError):
         ctx.relax_with_report(m, L.LLGParams(), lm, L.FieldMask.Full,
                               L.relax_settings(dt_min=1e-10, dt_max=1e-12))
+
+
+@pytest.mark.parametrize("prec,path", [("f32", "fft_fused"), ("f32", "fft_unfused"), ("f64", "fft_fused"),
+                                       ("f64", "no_demag"), ("f64", "mg")])
+def test_rk23_stage_epilogue_equals_stage_kernels(gpu_lib, prec, path, monkeypatch):
+    """Stage states 3 and 4 formed in the field evaluation's epilogue (the
+    default) against stage kernels of their own (LLGMI_RK45_FUSE=0): state, eps,
+    accept, dt and the kept field bitwise equal over 8 attempts, one rejected."""
+    from conftest import DeviceBuffer
+    from initial_states import smoothed_random
+    L = gpu_lib
+    P, es = (L.F32, 4) if prec == "f32" else (L.F64, 8)
+    nx, ny = 45, 21
+    mat = L.Material(ms=8e5, a_ex=1.3e-11, k_u=2e4, dmi=1e-3, demag=path != "no_demag")
+    if path == "mg":
+        mat.demag_method = L.DemagMethod.PoissonMG
+    mask = 1 if path == "no_demag" else 2
+    monkeypatch.setenv("LLGMI_FFT_FUSED", "1" if path == "fft_fused" else "0")
+    ctxs = [L.Context(L.Grid2D(nx, ny, 3e-9, 3e-9, 2e-9), precision=P) for _ in range(2)]
+    bufs = [DeviceBuffer(3 * nx * ny * es) for _ in range(2)]
+    pars = [L.LLGParams(alpha=0.3, dt=1e-13, b_ext=(0.0, 0.01, 0.02)) for _ in range(2)]
+    for c, b in zip(ctxs, bufs):
+        c.dev_upload(smoothed_random(nx, ny, 5).reshape(-1, 3), b)
+    rejected = 0
+    for step in range(8):
+        if step == 4:
+            pars[0].dt = pars[1].dt = 5e-11
+        res = []
+        for i in range(2):
+            if i == 0:
+                monkeypatch.delenv("LLGMI_RK45_FUSE", raising=False)
+            else:
+                monkeypatch.setenv("LLGMI_RK45_FUSE", "0")
+            res.append(ctxs[i].dev_rk23_relax_step(bufs[i], pars[i], mat, mask, 1e-5, 0.8, 1e-18, 1e-9))
+        assert res[0] == res[1] and pars[0].dt == pars[1].dt, step
+        assert np.array_equal(ctxs[0].dev_download(bufs[0]), ctxs[1].dev_download(bufs[1])), step
+        rejected += not res[0][1]
+    assert rejected >= 1
+    fields = [c.rk23_last_b_eff() for c in ctxs]
+    assert (fields[0] is None) == (fields[1] is None)
+    if fields[0] is not None:
+        assert np.array_equal(fields[0], fields[1])
