@@ -1094,6 +1094,28 @@ __device__ __forceinline__ void cell_pos(const BoxGeom &g, int i, int j, int k, 
     z = ((double)k + 0.5 - g.cz) * g.dz;
 }
 
+// q / sqrt(x) for x > 0.  The square root by one Goldschmidt step from the
+// hardware's reciprocal square root and two residual corrections; the same step
+// leaves half its reciprocal, so the quotient needs no division: one Newton step
+// makes that reciprocal good to the last place and a residual correction rounds
+// the quotient (both roundings those of sqrt and /, up to rare last-place cases
+// near a tie).  About 17 instructions against 32 for the two sequences; boundary
+// evaluation of the 512 x 512 hole lattice 1.92 -> 1.51 ms.
+__device__ __forceinline__ double div_sqrt(double q, double x) {
+    if (!(x > 0x1p-900 && x < 0x1p900)) return q / sqrt(x);
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    const double e = __builtin_fma(-h, g, 0.5);
+    g = __builtin_fma(g, e, g);
+    h = __builtin_fma(h, e, h);
+    g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+    g = __builtin_fma(__builtin_fma(-g, g, x), h, g);   // sqrt(x)
+    double r = h + h;
+    r = __builtin_fma(__builtin_fma(-r, g, 1.0), r, r);   // 1 / sqrt(x)
+    const double v = q * r;
+    return __builtin_fma(__builtin_fma(-v, g, q), r, v);
+}
+
 // eval_phi (mg_treecode.rs:192-259) at every boundary cell; writes bc and
 // stamps phi.  The boundary cells come in 8 x 8 patches of one face per wave
 // (targets, -1 = idle lane), so a wave's cells are close together.
@@ -1142,7 +1164,7 @@ __global__ void __launch_bounds__(kNT) k_tc_eval(const TNode *__restrict__ nodes
                     const double ex = tx - pos[3 * (int64_t)a], ey = ty - pos[3 * (int64_t)a + 1],
                                  ez = tz - pos[3 * (int64_t)a + 2];
                     const double rr2 = ex * ex + ey * ey + ez * ez;
-                    if (rr2 > 0.0) v += qp[a] / sqrt(rr2);
+                    if (rr2 > 0.0) v += div_sqrt(qp[a], rr2);
                 }
             } else {
                 const double rx = tx - nd.cx, ry = ty - nd.cy, rz = tz - nd.cz;
@@ -1163,8 +1185,7 @@ __global__ void __launch_bounds__(kNT) k_tc_eval(const TNode *__restrict__ nodes
                     accept = false;
                 }
                 if (accept) {
-                    const double r = sqrt(rx * rx + ry * ry + rz * rz);
-                    const double inv_r = 1.0 / r;
+                    const double inv_r = div_sqrt(1.0, rx * rx + ry * ry + rz * rz);
                     const double inv_r3 = inv_r * inv_r * inv_r;
                     const double pr = mom[4 * (int64_t)n + 1] * rx + mom[4 * (int64_t)n + 2] * ry +
                                       mom[4 * (int64_t)n + 3] * rz;
