@@ -50,8 +50,14 @@ namespace llgmi {
 __host__ __device__ constexpr int clampi(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); }
 __host__ __device__ constexpr int mini(int a, int b) { return a < b ? a : b; }
 
-// Row blocks: as many row pairs as fit the LDS / thread budget (more pairs per
-// block = longer contiguous runs in the column-major spectrum).
+// Row blocks: as many row pairs as give a store into the column-major spectrum
+// its full width (64 contiguous bytes: four pairs in FP32, two in FP64; narrower
+// runs store slower, wider ones no faster) and a block at least one wave.  More
+// pairs only make fewer, larger blocks, which leaves small grids on a handful
+// of CUs: at 128 x 64 in FP64 18 pairs per block meant 6 blocks.
+// (now 16): row passes of an RK45 attempt there 10 and 16 us -> 6 and 12 us with
+// radix 8, the attempt 245 -> 165 us; 64 films of 64..512 x 64..256, whose small
+// ones take radix 8 too, 10.9 -> 9.9 ms per 8 attempts; 1024^2 and 2048^2 unchanged.
 #ifndef LLGMI_ROW_LDS_KB
 #define LLGMI_ROW_LDS_KB 80
 #endif
@@ -59,11 +65,22 @@ __host__ __device__ constexpr int mini(int a, int b) { return a < b ? a : b; }
 #define LLGMI_ROW_NT 512
 #endif
 template <typename T, int LOG2L, int RQ = 0>
-struct RowCfg {
+struct BatchRowCfg {
+    // the batched passes take all that fit the LDS / thread budget: films of
+    // different lengths then have blocks of one shape and share a launch
     using P = Plan<LOG2L, RQ>;
     static constexpr int L = P::L, TPS = P::TPS, SLEN = lds_seq_len(L);
     static constexpr int PAIRS = clampi(mini((int)(LLGMI_ROW_LDS_KB * 1024 / (sizeof(cpx<T>) * SLEN)),
                                              LLGMI_ROW_NT / TPS), 1, 64);
+    static constexpr int NT = PAIRS * TPS;
+    static constexpr size_t LDS = sizeof(cpx<T>) * PAIRS * SLEN;
+};
+template <typename T, int LOG2L, int RQ = 0>
+struct RowCfg {
+    using P = Plan<LOG2L, RQ>;
+    static constexpr int L = P::L, TPS = P::TPS, SLEN = lds_seq_len(L);
+    static constexpr int FULL = 16 / (int)sizeof(T);   // pairs of a 64-byte run
+    static constexpr int PAIRS = mini(BatchRowCfg<T, LOG2L, RQ>::PAIRS, TPS >= 64 / FULL ? FULL : 64 / TPS);
     static constexpr int NT = PAIRS * TPS;
     static constexpr size_t LDS = sizeof(cpx<T>) * PAIRS * SLEN;
 };
@@ -103,11 +120,10 @@ struct ExtractCfg {
 // ---------------------------------------------------------------------------
 // HALF: ncols_valid == L/2, so the upper half of every row is a compile-time zero.
 // The block of component comp whose first row is j0.
-template <typename T, typename Tin, int LOG2L, bool HALF, int RQ>
+template <typename T, typename Tin, int LOG2L, bool HALF, int RQ, typename C = RowCfg<T, LOG2L, RQ>>
 __device__ __forceinline__ void row_r2c_body(const Tin *__restrict__ src, int64_t src_cstride, int row_stride,
                                              int ncols_valid, int nrows, T scale, const cpx<T> *__restrict__ tw,
                                              cpx<T> *__restrict__ dst, int64_t dst_cstride, int comp, int j0) {
-    using C = RowCfg<T, LOG2L, RQ>;
     using PL = typename C::P;
     constexpr int L = C::L, PAIRS = C::PAIRS, NT = C::NT, SLEN = C::SLEN, TPS = C::TPS;
     constexpr int NV = PL::NV;
@@ -470,11 +486,10 @@ k_colsplit_mul_inv(cpx<T> *__restrict__ S, const cpx<T> *__restrict__ F, int hxs
 // ---------------------------------------------------------------------------
 // HALF: nx == L/2, so only the lower half of each inverse-transformed row is
 // formed and stored.
-template <typename T, int LOG2L, bool HALF, int RQ>
+template <typename T, int LOG2L, bool HALF, int RQ, typename C = RowCfg<T, LOG2L, RQ>>
 __device__ __forceinline__ void row_c2r_body(const cpx<T> *__restrict__ S, int hxs, int nx, int ny,
                                              const cpx<T> *__restrict__ tw, T *__restrict__ out, int64_t n,
                                              int comp, int j0) {
-    using C = RowCfg<T, LOG2L, RQ>;
     using PL = typename C::P;
     constexpr int L = C::L, PAIRS = C::PAIRS, NT = C::NT, SLEN = C::SLEN, TPS = C::TPS;
     constexpr int NV = PL::NV;
@@ -1484,17 +1499,21 @@ void DemagFFT<T>::launch_row_inv(T *bd, hipStream_t stream, int rq) {
 // Per grid, time the radix-8 and radix-16 variants of each pass and keep the
 // faster: which one wins depends on the lengths through occupancy (registers)
 // versus LDS round trips.  LLGMI_FFT_RADIX=8 or 16 forces one variant for all
-// passes (used by tests to cover both); grids below 256 x 256 padded points
-// are launch-bound and keep radix 16 without timing.
+// passes (used by tests to cover both); grids below 256 x 256 padded points are
+// bound by the latency of one thread's chain, not by its arithmetic, and take
+// radix 8 without timing (half the values per thread: an RK45 attempt at 128 x 64
+// in FP64 206 us against 224 us with radix 16).
 template <typename T>
 void DemagFFT<T>::autotune(hipStream_t stream, int forced) {
     // LLGMI_FFT_COLPIPE=0|1 forces the one-item-per-block or the persistent
     // column pass
     const char *pe = std::getenv("LLGMI_FFT_COLPIPE");
     const int pipe_forced = pe ? (pe[0] == '1' ? 1 : 0) : -1;
-    rq_row = rq_col = rq_row_inv = forced ? forced : 4;
+    const bool small = px * py < 256 * 256;
+    // (the longest transforms are built for radix 16 in every pass)
+    rq_row = rq_col = rq_row_inv = forced ? forced : small && px <= 2048 && py <= 2048 ? 3 : 4;
     if (pipe_forced == 1) rq_col |= kColPipe;
-    if (forced || px * py < 256 * 256) return;
+    if (forced || small) return;
     const bool shared = pipe_forced < 0;   // forced settings neither read nor set the shared choice
     const TuneKey key = tune_key(*this);
     if (shared) {
@@ -1666,7 +1685,7 @@ void DemagFFT<T>::field_local(const T *m, T ms, const LocalArgs<T> &a, const uin
         } else if (fv == "1") {
             rq_fused = fits(rq_row_inv) ? rq_row_inv : (fits(3) ? 3 : (fits(4) ? 4 : -1));
         } else if (px * py < 256 * 256) {
-            rq_fused = fits(4) ? 4 : (fits(3) ? 3 : -1);
+            rq_fused = fits(rq_row_inv) ? rq_row_inv : (fits(3) ? 3 : (fits(4) ? 4 : -1));
         } else {
             const std::pair<TuneKey, int> fkey{tune_key(*this), rq_row_inv};
             {
@@ -1732,8 +1751,8 @@ struct BatchCfg;
 template <typename T, int LG, int RQ>
 struct BatchCfg<T, 0, LG, RQ> {
     static constexpr bool OK = LG >= 1 && LG <= Range<T>::ROW;
-    static constexpr int NT = RowCfg<T, LG, RQ>::NT;
-    static constexpr size_t LDS = RowCfg<T, LG, RQ>::LDS;
+    static constexpr int NT = BatchRowCfg<T, LG, RQ>::NT;
+    static constexpr size_t LDS = BatchRowCfg<T, LG, RQ>::LDS;
 };
 template <typename T, int LG, int RQ>
 struct BatchCfg<T, 2, LG, RQ> : BatchCfg<T, 0, LG, RQ> {};
@@ -1797,17 +1816,18 @@ __device__ __forceinline__ void dev_dispatch_log2(int lg, Fn &&fn) {
 }
 
 template <typename T, int LO, int HI, bool HALF, int RQ>
-__global__ void __launch_bounds__((RowCfg<T, LO, RQ>::NT))
+__global__ void __launch_bounds__((BatchRowCfg<T, LO, RQ>::NT))
 kb_row_r2c(const BFilm<T> *__restrict__ F, const BEntry *__restrict__ tab, int which, int stage1) {
     const BEntry e = tab[blockIdx.x];
     const BFilm<T> &f = F[e.film];
     if (stage1 && f.skip1) return;
     dev_dispatch_log2<LO, HI>(__builtin_ctz((unsigned)f.px), [&](auto lgc) {
         constexpr int LG = decltype(lgc)::value;
-        constexpr int PAIRS = RowCfg<T, LG, RQ>::PAIRS;
+        using C = BatchRowCfg<T, LG, RQ>;
+        constexpr int PAIRS = C::PAIRS;
         const int nb = (f.ny + 2 * PAIRS - 1) / (2 * PAIRS);
         const int comp = e.blk / nb, j0 = (e.blk - comp * nb) * 2 * PAIRS;
-        row_r2c_body<T, T, LG, HALF, RQ>(f.in[which], (int64_t)f.nx * f.ny, f.nx, f.nx, f.ny, f.ms, f.tw_x, f.spec,
+        row_r2c_body<T, T, LG, HALF, RQ, C>(f.in[which], (int64_t)f.nx * f.ny, f.nx, f.nx, f.ny, f.ms, f.tw_x, f.spec,
                                          (int64_t)(f.px / 2) * f.ny, comp, j0);
     });
 }
@@ -1826,17 +1846,18 @@ kb_col(const BFilm<T> *__restrict__ F, const BEntry *__restrict__ tab, int stage
 }
 
 template <typename T, int LO, int HI, bool HALF, int RQ>
-__global__ void __launch_bounds__((RowCfg<T, LO, RQ>::NT))
+__global__ void __launch_bounds__((BatchRowCfg<T, LO, RQ>::NT))
 kb_row_c2r(const BFilm<T> *__restrict__ F, const BEntry *__restrict__ tab, int stage1) {
     const BEntry e = tab[blockIdx.x];
     const BFilm<T> &f = F[e.film];
     if (stage1 && f.skip1) return;
     dev_dispatch_log2<LO, HI>(__builtin_ctz((unsigned)f.px), [&](auto lgc) {
         constexpr int LG = decltype(lgc)::value;
-        constexpr int PAIRS = RowCfg<T, LG, RQ>::PAIRS;
+        using C = BatchRowCfg<T, LG, RQ>;
+        constexpr int PAIRS = C::PAIRS;
         const int nb = (f.ny + 2 * PAIRS - 1) / (2 * PAIRS);
         const int comp = e.blk / nb, j0 = (e.blk - comp * nb) * 2 * PAIRS;
-        row_c2r_body<T, LG, HALF, RQ>(f.spec, f.px / 2, f.nx, f.ny, f.tw_x, f.bd, (int64_t)f.nx * f.ny, comp, j0);
+        row_c2r_body<T, LG, HALF, RQ, C>(f.spec, f.px / 2, f.nx, f.ny, f.tw_x, f.bd, (int64_t)f.nx * f.ny, comp, j0);
     });
 }
 
@@ -1875,7 +1896,7 @@ int batch_row_blocks(int kind, int lg, int rq, int ny) {
         if (kind == 3) {
             pairs = rq == 3 ? BatchFusedCfg<T, LG, 3>::PAIRS : BatchFusedCfg<T, LG, 4>::PAIRS;
         } else {
-            pairs = rq == 3 ? RowCfg<T, LG, 3>::PAIRS : RowCfg<T, LG, 4>::PAIRS;
+            pairs = rq == 3 ? BatchRowCfg<T, LG, 3>::PAIRS : BatchRowCfg<T, LG, 4>::PAIRS;
         }
     });
     return (ny + 2 * pairs - 1) / (2 * pairs);

@@ -549,3 +549,47 @@ def test_fft_pad_env_rejects_other_values(gpu_lib, monkeypatch):
     with pytest.raises(L.LlgmiError) as e:
         ctx.compute_demag_field(_rand_m(256, 1), L.Material(ms=8e5, demag=True))
     assert e.value.code == L.ERR_INVALID
+
+
+# Both sides of the lines at which a grid takes radix 8 without timing (fewer
+# than 256 x 256 padded points, transforms of at most 2048), and row blocks of
+# one pair, remainders and single rows: the field against the oracle, and one
+# batched attempt of all of them bitwise as stepped alone.
+SMALL = [(128, 64), (128, 128), (1024, 7), (1030, 4), (2, 1030), (2, 2100), (33, 1), (61, 37)]
+
+
+@pytest.mark.parametrize("nx,ny", SMALL)
+@pytest.mark.parametrize("prec", ["f32", "f64"])
+def test_small_grid_radix_and_row_blocks(gpu_lib, nx, ny, prec):
+    L = gpu_lib
+    cell = (3e-9, 4e-9, 3e-9)
+    rng = np.random.default_rng(nx + ny)
+    m = rng.standard_normal((nx * ny, 3))
+    m /= np.linalg.norm(m, axis=1, keepdims=True)
+    want = np.zeros_like(m)
+    from oracle import oracle as O
+    O.Context(O.Grid(nx, ny, *cell)).add_demag(m, want, O.Material(ms=8e5, demag=True))
+    ctx = L.Context(L.Grid2D(nx, ny, *cell), precision=L.F32 if prec == "f32" else L.F64)
+    got = ctx.compute_demag_field(m, L.Material(ms=8e5, demag=True))
+    assert rel_err(got, want) <= (1e-5 if prec == "f32" else 1e-12)
+
+
+def test_small_grids_batched_as_alone(gpu_lib):
+    from conftest import DeviceBuffer
+    L = gpu_lib
+    alone, batch = [], []
+    for out in (alone, batch):
+        for nx, ny in SMALL:
+            c = L.Context(L.Grid2D(nx, ny, 3e-9, 4e-9, 3e-9), precision=L.F32)
+            m = np.random.default_rng(nx + ny).standard_normal((nx * ny, 3))
+            m /= np.linalg.norm(m, axis=1, keepdims=True)
+            b = DeviceBuffer(3 * nx * ny * 4)
+            c.dev_upload(m, b)
+            out.append((c, b, L.LLGParams(alpha=0.1, dt=1e-14, b_ext=(0.0, 0.0, 0.01)),
+                        L.Material(ms=8e5, a_ex=1.3e-11, demag=True)))
+    rk = dict(mask=L.FieldMask.Full, max_err=1e-5, headroom=0.8, dt_min=1e-18, dt_max=1e-11)
+    for _ in range(3):
+        r = L.dev_rk45_step_batch(*[[x[k] for x in batch] for k in range(4)], **rk)
+        for i, (c, b, p, mat) in enumerate(alone):
+            assert c.dev_rk45_step(b, p, mat, **rk) == r[i], SMALL[i]
+            assert np.array_equal(c.dev_download(b), batch[i][0].dev_download(batch[i][1])), SMALL[i]
