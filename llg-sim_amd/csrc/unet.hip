@@ -11,8 +11,7 @@
 // zero or from the previous solve, demag_poisson_mg.rs:1947-2057).
 //
 // Layout: activations channels-last, pixel p = (b*H + y)*W + x for batch b,
-// row y, column x; a tensor slice is (pointer, channel stride, channel
-// offset).  Convolution weights [tap][c_out][c_in] with tap = (dy+1)*3+(dx+1),
+// row y, column x, every tensor dense.  Convolution weights [tap][c_out][c_in] with tap = (dy+1)*3+(dx+1),
 // zero padding at the image border.
 //
 // Architecture (levels l = 0..3, c_l = base * 2^l):

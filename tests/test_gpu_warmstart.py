@@ -6,11 +6,8 @@
   device accumulates in FP32 (the oracle in float64), so a bf16 rounding can
   land on the other side in a few elements: the bars are relative L2 norms,
   forward 1e-5 (measured 6e-8), each layer's gradient 1e-3 (worst measured
-  7e-4), all gradients 3e-4 (measured 1.05e-4).  The spatial-tile
-  convolutions (the default) sum 32 channels per matrix-core instruction;
-  the pixel-row kernel (LLGMI_UNET_TILE=0, 16 per instruction) lands closer
-  to the emulation's roundings (4e-5 worst layer, 3.6e-6 in all), and
-  against float64 the two are equally accurate (the large-plane test).
+  7e-4), all gradients 3e-4 (measured 1.05e-4).  LLGMI_UNET_TILE=0 takes the
+  smallest pixel tile at every level.
 * Adam training on the device reduces the loss of a learnable map.
 * The trained network's potential, written into the multigrid solver as its
   initial phi, reaches the same residual in fewer V-cycles than the zero
