@@ -530,13 +530,25 @@ __global__ void __launch_bounds__(TB_NT) k_mg_rb_tb(const double *__restrict__ A
     }
 }
 
-// Cell of a thread of the grids below (blocks of 64 x 4 cells of one plane, one
-// plane per blockIdx.z): no division per cell.
-constexpr int kBX = 64, kBY = 4;
-__device__ __forceinline__ int cell_i() { return (int)(blockIdx.x * kBX + threadIdx.x); }
-__device__ __forceinline__ int cell_j() { return (int)(blockIdx.y * kBY + threadIdx.y); }
+// Cells of the grids below (blocks of 64 x 4 cells of one plane, one plane per
+// blockIdx.z): no division per cell.  Rows and planes beyond the grid's limits
+// are strided over.
+constexpr int kBX = 64, kBY = 4, kGridMax = 65535;
 inline dim3 cell_grid(int nx, int ny, int nz) {
-    return dim3((unsigned)((nx + kBX - 1) / kBX), (unsigned)((ny + kBY - 1) / kBY), (unsigned)nz);
+    return dim3((unsigned)((nx + kBX - 1) / kBX), (unsigned)std::min((ny + kBY - 1) / kBY, kGridMax),
+                (unsigned)std::min(nz, kGridMax));
+}
+template <typename F>
+__device__ __forceinline__ void for_cells(int nx, int ny, int nz, F &&f) {
+    const int i = (int)(blockIdx.x * kBX + threadIdx.x);
+    if (i >= nx) return;
+    int j = (int)(blockIdx.y * kBY + threadIdx.y);
+    if (gridDim.y < kGridMax && gridDim.z < kGridMax) {   // one cell per thread (a loop costs 2 % of a solve)
+        if (j < ny) f(i, j, (int)blockIdx.z);
+        return;
+    }
+    for (int k = (int)blockIdx.z; k < nz; k += (int)gridDim.z)
+        for (j = (int)(blockIdx.y * kBY + threadIdx.y); j < ny; j += (int)gridDim.y * kBY) f(i, j, k);
 }
 
 // One sweep of smooth_weighted_jacobi from src into dst; boundary cells of dst
@@ -545,19 +557,19 @@ __global__ void __launch_bounds__(kBX *kBY) k_mg_wj(const double *__restrict__ s
                                                     const double *__restrict__ rhs, const double *__restrict__ bc,
                                                     const DevStencil *__restrict__ st, ExactDiv diag, double omega,
                                                     int nx, int ny, int nz) {
-    const int i = cell_i(), j = cell_j(), k = (int)blockIdx.z;
-    if (i >= nx || j >= ny) return;
-    const int64_t id = idx3(i, j, k, nx, ny);
-    if (i == 0 || i == nx - 1 || j == 0 || j == ny - 1 || k == 0 || k == nz - 1) {
-        dst[id] = bc ? bc[id] : 0.0;
-        return;
-    }
-    const double off = offdiag_in(src, id, nx, ny, nz, i, j, k, st);
-    const double s = src[id];
-    double gs[1] = {off - rhs[id]};
-    if (fabs(diag.d) > 1e-30) div_by(gs, diag);
-    else gs[0] = s;
-    dst[id] = (1.0 - omega) * s + omega * gs[0];
+    for_cells(nx, ny, nz, [&](int i, int j, int k) {
+        const int64_t id = idx3(i, j, k, nx, ny);
+        if (i == 0 || i == nx - 1 || j == 0 || j == ny - 1 || k == 0 || k == nz - 1) {
+            dst[id] = bc ? bc[id] : 0.0;
+            return;
+        }
+        const double off = offdiag_in(src, id, nx, ny, nz, i, j, k, st);
+        const double s = src[id];
+        double gs[1] = {off - rhs[id]};
+        if (fabs(diag.d) > 1e-30) div_by(gs, diag);
+        else gs[0] = s;
+        dst[id] = (1.0 - omega) * s + omega * gs[0];
+    });
 }
 
 // `nsweep` weighted-Jacobi sweeps in one launch, for small levels of at most
@@ -690,22 +702,23 @@ __global__ void __launch_bounds__(kBX *kBY) k_mg_resid_restrict(const double *__
                                                            double *__restrict__ cphi, int cnx, int cny,
                                                            int cnz, int rx, int ry, int rz, double w,
                                                            int seven) {
-    const int ic = 1 + cell_i(), jc = 1 + cell_j(), kc = 1 + (int)blockIdx.z;
-    if (ic > cnx - 2 || jc > cny - 2) return;
-    double sum = 0.0;
-    for (int dk = 0; dk < rz; ++dk)
-        for (int dj = 0; dj < ry; ++dj)
-            for (int di = 0; di < rx; ++di) {
-                const int i = rx * ic + di, j = ry * jc + dj, k = rz * kc + dk;
-                const int64_t id = idx3(i, j, k, fnx, fny);
-                const double a = st->center * phi[id] +
-                                 (seven ? offdiag7(phi, id, fnx, (int64_t)fnx * fny, st)
-                                        : offdiag_in(phi, id, fnx, fny, fnz, i, j, k, st));
-                sum += rhs[id] - a;
-            }
-    const int64_t cid = idx3(ic, jc, kc, cnx, cny);
-    crhs[cid] = w * sum;
-    cphi[cid] = 0.0;
+    for_cells(cnx - 2, cny - 2, cnz - 2, [&](int ci, int cj, int ck) {
+        const int ic = 1 + ci, jc = 1 + cj, kc = 1 + ck;
+        double sum = 0.0;
+        for (int dk = 0; dk < rz; ++dk)
+            for (int dj = 0; dj < ry; ++dj)
+                for (int di = 0; di < rx; ++di) {
+                    const int i = rx * ic + di, j = ry * jc + dj, k = rz * kc + dk;
+                    const int64_t id = idx3(i, j, k, fnx, fny);
+                    const double a = st->center * phi[id] +
+                                     (seven ? offdiag7(phi, id, fnx, (int64_t)fnx * fny, st)
+                                            : offdiag_in(phi, id, fnx, fny, fnz, i, j, k, st));
+                    sum += rhs[id] - a;
+                }
+        const int64_t cid = idx3(ic, jc, kc, cnx, cny);
+        crhs[cid] = w * sum;
+        cphi[cid] = 0.0;
+    });
 }
 
 __device__ __forceinline__ void interp_1d(int ic, int ri, int nc, int r, int &i0o, int &i1o, double &w0,
@@ -734,30 +747,31 @@ __device__ __forceinline__ void interp_1d(int ic, int ri, int nc, int r, int &i0
 __global__ void __launch_bounds__(kBX *kBY) k_mg_prolong(const double *__restrict__ c, int cnx, int cny, int cnz,
                                                     double *__restrict__ f, int fnx, int fny, int fnz,
                                                     int trilinear) {
-    const int i = 1 + cell_i(), j = 1 + cell_j(), k = 1 + (int)blockIdx.z;
-    if (i > fnx - 2 || j > fny - 2) return;
-    const int rx = fnx / cnx, ry = fny / cny, rz = fnz / cnz;
-    const int64_t id = idx3(i, j, k, fnx, fny);
-    if (trilinear) {
-        int k0, k1, j0, j1, i0, i1;
-        double wk0, wk1, wj0, wj1, wi0, wi1;
-        interp_1d(k / rz, k % rz, cnz, rz, k0, k1, wk0, wk1);
-        interp_1d(j / ry, j % ry, cny, ry, j0, j1, wj0, wj1);
-        interp_1d(i / rx, i % rx, cnx, rx, i0, i1, wi0, wi1);
-        const double v = wi0 * wj0 * wk0 * c[idx3(i0, j0, k0, cnx, cny)]
-                       + wi1 * wj0 * wk0 * c[idx3(i1, j0, k0, cnx, cny)]
-                       + wi0 * wj1 * wk0 * c[idx3(i0, j1, k0, cnx, cny)]
-                       + wi1 * wj1 * wk0 * c[idx3(i1, j1, k0, cnx, cny)]
-                       + wi0 * wj0 * wk1 * c[idx3(i0, j0, k1, cnx, cny)]
-                       + wi1 * wj0 * wk1 * c[idx3(i1, j0, k1, cnx, cny)]
-                       + wi0 * wj1 * wk1 * c[idx3(i0, j1, k1, cnx, cny)]
-                       + wi1 * wj1 * wk1 * c[idx3(i1, j1, k1, cnx, cny)];
-        f[id] += v;
-    } else {
-        const int ic = i / rx, jc = j / ry, kc = k / rz;
-        if (ic == 0 || ic + 1 >= cnx || jc == 0 || jc + 1 >= cny || kc == 0 || kc + 1 >= cnz) return;
-        f[id] += c[idx3(ic, jc, kc, cnx, cny)];
-    }
+    for_cells(fnx - 2, fny - 2, fnz - 2, [&](int fi, int fj, int fk) {
+        const int i = 1 + fi, j = 1 + fj, k = 1 + fk;
+        const int rx = fnx / cnx, ry = fny / cny, rz = fnz / cnz;
+        const int64_t id = idx3(i, j, k, fnx, fny);
+        if (trilinear) {
+            int k0, k1, j0, j1, i0, i1;
+            double wk0, wk1, wj0, wj1, wi0, wi1;
+            interp_1d(k / rz, k % rz, cnz, rz, k0, k1, wk0, wk1);
+            interp_1d(j / ry, j % ry, cny, ry, j0, j1, wj0, wj1);
+            interp_1d(i / rx, i % rx, cnx, rx, i0, i1, wi0, wi1);
+            const double v = wi0 * wj0 * wk0 * c[idx3(i0, j0, k0, cnx, cny)]
+                           + wi1 * wj0 * wk0 * c[idx3(i1, j0, k0, cnx, cny)]
+                           + wi0 * wj1 * wk0 * c[idx3(i0, j1, k0, cnx, cny)]
+                           + wi1 * wj1 * wk0 * c[idx3(i1, j1, k0, cnx, cny)]
+                           + wi0 * wj0 * wk1 * c[idx3(i0, j0, k1, cnx, cny)]
+                           + wi1 * wj0 * wk1 * c[idx3(i1, j0, k1, cnx, cny)]
+                           + wi0 * wj1 * wk1 * c[idx3(i0, j1, k1, cnx, cny)]
+                           + wi1 * wj1 * wk1 * c[idx3(i1, j1, k1, cnx, cny)];
+            f[id] += v;
+        } else {
+            const int ic = i / rx, jc = j / ry, kc = k / rz;
+            if (ic == 0 || ic + 1 >= cnx || jc == 0 || jc + 1 >= cny || kc == 0 || kc + 1 >= cnz) return;
+            f[id] += c[idx3(ic, jc, kc, cnx, cny)];
+        }
+    });
 }
 
 // Dirichlet stamp of the boundary cells (stamp_dirichlet_bc, mg_kernels.rs:35-61)
@@ -2236,16 +2250,18 @@ void MGSolver::smooth(int l, int64_t iters) {
         auto blocks = [&](int T) { return (int64_t)((L.nx - 2 + T - 1) / T) * ((L.ny - 2 + T - 1) / T); };
         int T = 4;
         while (T < WJW - 4 && blocks(T) > 256) T += 2;
-        const dim3 grid((unsigned)((L.nx - 2 + T - 1) / T), (unsigned)((L.ny - 2 + T - 1) / T));
-        for (int64_t left = iters; left > 0;) {
-            const int h = (int)std::min<int64_t>(left, (WJW - T) / 2);
-            hipLaunchKernelGGL(k_mg_wj_tb, grid, dim3(WJW * WJW), 0, stream_, L.phi[L.cur], L.phi[1 - L.cur], L.rhs,
-                               L.nx, L.ny, L.nz, co, diag, cfg_.omega, h, T);
-            LLGMI_LAUNCH_CHECK();
-            L.cur = 1 - L.cur;
-            left -= h;
+        if ((L.ny - 2 + T - 1) / T <= kGridMax) {
+            const dim3 grid((unsigned)((L.nx - 2 + T - 1) / T), (unsigned)((L.ny - 2 + T - 1) / T));
+            for (int64_t left = iters; left > 0;) {
+                const int h = (int)std::min<int64_t>(left, (WJW - T) / 2);
+                hipLaunchKernelGGL(k_mg_wj_tb, grid, dim3(WJW * WJW), 0, stream_, L.phi[L.cur], L.phi[1 - L.cur], L.rhs,
+                                   L.nx, L.ny, L.nz, co, diag, cfg_.omega, h, T);
+                LLGMI_LAUNCH_CHECK();
+                L.cur = 1 - L.cur;
+                left -= h;
+            }
+            return;
         }
-        return;
     }
     for (int64_t it = 0; it < iters; ++it) {
         hipLaunchKernelGGL(k_mg_wj, cell_grid(L.nx, L.ny, L.nz), dim3(kBX, kBY), 0, stream_, L.phi[L.cur],

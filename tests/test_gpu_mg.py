@@ -65,10 +65,11 @@ def test_mg_fp64_matches_oracle_with_warm_start(gpu_lib, op, bc):
 # boundary: two-sweep boxes of 32 x 16 (24 x 8 columns) with one, full and
 # remainder tiles, odd sweep counts (the last one in place), coarsest levels of
 # nine and fewer planes and of several tiles, a flat box and one that does not
-# coarsen in the plane; 640 x 600 takes the 64 x 32 boxes.
+# coarsen in the plane; 640 x 600 takes the 64 x 32 boxes; 270000 rows exceed
+# the launch grid's second dimension.
 @pytest.mark.parametrize("nx,ny,nvac,pre,post,cycles", [
     (7, 5, 3, 2, 2, 3), (26, 10, 4, 2, 1, 3), (27, 41, 8, 3, 2, 3), (50, 34, 16, 1, 4, 3), (75, 12, 16, 2, 3, 3),
-    (131, 90, 5, 2, 2, 2), (640, 600, 2, 2, 2, 1)])
+    (131, 90, 5, 2, 2, 2), (640, 600, 2, 2, 2, 1), (1, 270000, 2, 2, 2, 1)])
 @pytest.mark.parametrize("op", ["rb7_inject_rd", "iso27_tri_galerkin"])
 def test_mg_smoother_tile_edges(gpu_lib, nx, ny, nvac, pre, post, cycles, op):
     from oracle import oracle as O
