@@ -56,8 +56,7 @@ __host__ __device__ constexpr int mini(int a, int b) { return a < b ? a : b; }
 // pairs only make fewer, larger blocks, which leaves small grids on a handful
 // of CUs: at 128 x 64 in FP64 18 pairs per block meant 6 blocks.
 // (now 16): row passes of an RK45 attempt there 10 and 16 us -> 6 and 12 us with
-// radix 8, the attempt 245 -> 165 us; 64 films of 64..512 x 64..256, whose small
-// ones take radix 8 too, 10.9 -> 9.9 ms per 8 attempts; 1024^2 and 2048^2 unchanged.
+// radix 8, the attempt 245 -> 165 us; 1024^2 and 2048^2 unchanged.
 #ifndef LLGMI_ROW_LDS_KB
 #define LLGMI_ROW_LDS_KB 80
 #endif
@@ -1499,10 +1498,14 @@ void DemagFFT<T>::launch_row_inv(T *bd, hipStream_t stream, int rq) {
 // Per grid, time the radix-8 and radix-16 variants of each pass and keep the
 // faster: which one wins depends on the lengths through occupancy (registers)
 // versus LDS round trips.  LLGMI_FFT_RADIX=8 or 16 forces one variant for all
-// passes (used by tests to cover both); grids below 256 x 256 padded points are
-// bound by the latency of one thread's chain, not by its arithmetic, and take
-// radix 8 without timing (half the values per thread: an RK45 attempt at 128 x 64
-// in FP64 206 us against 224 us with radix 16).
+// passes (used by tests to cover both).  Grids below 256 x 256 padded points are
+// not timed.  They are bound by the latency of one thread's chain, which radix 8
+// shortens (half the values per thread: an RK45 attempt at 128 x 64 in FP64 takes
+// 163 us against 233 us with radix 16), but its third stage at 256 points costs
+// accuracy: in FP32 the field is 10 to 19 % further from an 80-bit convolution than
+// with radix 16, so FP32 keeps radix 16.  FP64 takes radix 8 up to 512 points, where
+// its twiddles all come from the table and it is the more accurate one
+// (reg_fft_rest).
 template <typename T>
 void DemagFFT<T>::autotune(hipStream_t stream, int forced) {
     // LLGMI_FFT_COLPIPE=0|1 forces the one-item-per-block or the persistent
@@ -1510,8 +1513,7 @@ void DemagFFT<T>::autotune(hipStream_t stream, int forced) {
     const char *pe = std::getenv("LLGMI_FFT_COLPIPE");
     const int pipe_forced = pe ? (pe[0] == '1' ? 1 : 0) : -1;
     const bool small = px * py < 256 * 256;
-    // (the longest transforms are built for radix 16 in every pass)
-    rq_row = rq_col = rq_row_inv = forced ? forced : small && px <= 2048 && py <= 2048 ? 3 : 4;
+    rq_row = rq_col = rq_row_inv = forced ? forced : small && sizeof(T) == 8 && px <= 512 && py <= 512 ? 3 : 4;
     if (pipe_forced == 1) rq_col |= kColPipe;
     if (forced || small) return;
     const bool shared = pipe_forced < 0;   // forced settings neither read nor set the shared choice

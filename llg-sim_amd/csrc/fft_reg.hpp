@@ -104,23 +104,38 @@ struct RegPlan {
 // Twiddles of stage (Ns, R) for butterfly class k: w^r with w = tw[k L/(Ns R)],
 // r < R.  Only w, w^4 and w^8 are gathered from the table, before the stage's
 // barrier so that the load latency overlaps the wait; the other powers are
-// products of at most three table values (a few ulp in FP32).
-template <typename T, int R>
+// products of at most three table values (a few ulp in FP32).  ALL: every power
+// from the table.
+template <typename T, int R, bool ALL>
 struct TwBase {
     cpx<T> w1, w4, w8;
 };
 template <typename T, int R>
-__device__ __forceinline__ TwBase<T, R> twiddle_load(const cpx<T> *__restrict__ tw, int base) {
-    TwBase<T, R> b;
-    b.w1 = tw[base];
-    if constexpr (R >= 8) b.w4 = tw[4 * base];
-    if constexpr (R == 16) b.w8 = tw[8 * base];
+struct TwBase<T, R, true> {
+    cpx<T> w[R];
+};
+template <typename T, int R, bool ALL>
+__device__ __forceinline__ TwBase<T, R, ALL> twiddle_load(const cpx<T> *__restrict__ tw, int base) {
+    TwBase<T, R, ALL> b;
+    if constexpr (ALL) {
+#pragma unroll
+        for (int r = 1; r < R; ++r) b.w[r] = tw[r * base];
+    } else {
+        b.w1 = tw[base];
+        if constexpr (R >= 8) b.w4 = tw[4 * base];
+        if constexpr (R == 16) b.w8 = tw[8 * base];
+    }
     return b;
 }
 // All powers w^r, r = 1..R-1, from the table values (formed once per stage
 // and thread, shared by the thread's butterflies of that stage).
 template <typename T, int R>
-__device__ __forceinline__ void twiddle_powers(const TwBase<T, R> &b, cpx<T> *w) {
+__device__ __forceinline__ void twiddle_powers(const TwBase<T, R, true> &b, cpx<T> *w) {
+#pragma unroll
+    for (int r = 1; r < R; ++r) w[r] = b.w[r];
+}
+template <typename T, int R>
+__device__ __forceinline__ void twiddle_powers(const TwBase<T, R, false> &b, cpx<T> *w) {
     w[1] = b.w1;
     if constexpr (R > 2) {
         w[2] = cmul(w[1], w[1]);
@@ -162,7 +177,13 @@ __device__ __forceinline__ void reg_fft_rest(cpx<T> *v, cpx<T> *seq, int t,
         constexpr int TWS = LOG2L - LOG2NS - LOG2R;
         constexpr bool LAST = LOG2NS + LOG2R == LOG2L;
         static_assert(TPS % NS == 0, "butterfly class must not depend on the butterfly");
-        const TwBase<T, R> twb = twiddle_load<T, R>(tw, (t & (NS - 1)) << TWS);
+        // 256 points take 8.4.8 with radix 8 against 16.16: with products for the
+        // powers the FP64 field is 3 to 9 % further from an 80-bit convolution, with
+        // every power from the table 5 to 7 % nearer, at the same speed.  Small FP64
+        // grids take radix 8 for its shorter chain, at 256 and 512 points.  (At 1024
+        // points the table's loads cost 4 % of an evaluation of 512 x 512.)
+        constexpr bool ALL = sizeof(T) == 8 && P::R0 == 8 && (LOG2L == 8 || LOG2L == 9);
+        const TwBase<T, R, ALL> twb = twiddle_load<T, R, ALL>(tw, (t & (NS - 1)) << TWS);
         __syncthreads();  // previous stage's LDS writes are visible
         const cpx<T> *rb = seq + lds_pad(t);
         cpx<T> w[R];
