@@ -1652,10 +1652,11 @@ void DemagFFT<T>::launch_row_inv_local(const LocalArgs<T> &a, const T *m, const 
     });
 }
 
-// First call on a grid: the fused pass (radix 8 or 16, where the block fits)
-// and the unfused pair (inverse row pass + local-field kernel) are timed on
-// the real arguments and the fastest kept.  LLGMI_FFT_FUSED=0 / 1 forces the
-// unfused / fused path (fused with the radix of the inverse row pass).
+// Small grids take the fused pass.  First call on any other grid: the fused pass
+// (radix 8 or 16, where the block fits) and the unfused pair (inverse row pass +
+// local-field kernel) are timed on the real arguments and the fastest kept.
+// LLGMI_FFT_FUSED=0 / 1 forces the unfused / fused path (fused with the radix of
+// the inverse row pass).
 template <typename T>
 void DemagFFT<T>::field_local(const T *m, T ms, const LocalArgs<T> &a, const uint8_t *geom, T *b, T *kout,
                               T *bd_scratch, hipStream_t stream, Profiler *prof) {
@@ -1686,7 +1687,12 @@ void DemagFFT<T>::field_local(const T *m, T ms, const LocalArgs<T> &a, const uin
             rq_fused = -1;
         } else if (fv == "1") {
             rq_fused = fits(rq_row_inv) ? rq_row_inv : (fits(3) ? 3 : (fits(4) ? 4 : -1));
-        } else if (px * py < 256 * 256) {
+        } else if (px * py < 256 * 256 || (sizeof(T) == 4 && px <= 512 && px * py <= 512 * 512)) {
+            // In FP32 the pair takes as long as the fused pass here (128 x 128 to
+            // 256 x 256 cells: 6.8 to 7.3 us against 6.7 to 7.0) and is one launch
+            // more, which a loop over many films waits for on the host (64 films on
+            // streams of their own: 950 us a round fused, 1040 us where timing the
+            // two found the pair faster).  In FP64 it is 0.5 to 1.2 us the faster.
             rq_fused = fits(rq_row_inv) ? rq_row_inv : (fits(3) ? 3 : (fits(4) ? 4 : -1));
         } else {
             const std::pair<TuneKey, int> fkey{tune_key(*this), rq_row_inv};
