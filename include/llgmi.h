@@ -331,7 +331,8 @@ int llgmi_mg_phi_write(llgmi_ctx *ctx, const double *phi_dev);
  * channels 0..3) to outputs y[b][y][x][c_pad] (FP32, c_pad = out_channels
  * rounded up to 16); trained on the device.  The loss is the mean squared
  * error over channels < out_channels and pixels x < valid_width,
- * y < valid_height, against bf16 targets t[b][y][x][c_pad]. */
+ * y < valid_height (beyond the plane: all of it), against bf16 targets
+ * t[b][y][x][c_pad]. */
 typedef struct llgmi_ws llgmi_ws;
 typedef struct llgmi_ws_shape {
     int64_t batch, height, width;       /* height, width multiples of 8 */

@@ -81,7 +81,8 @@ __device__ __forceinline__ uint4 src_load(const ConvSrc &s, int c, bool low, int
 //  MASK  bf16 of the sum where mask > 0, else 0, to y: a data gradient and the
 //        ReLU backward of the layer before it
 //  MSE   the loss's terms of sum + bias against tgt (channels < cv, pixels
-//        x < wv, y < hv) added to *loss, and the bf16 of the loss gradient to y
+//        x < wv <= W, y < hv <= H: a tile overhangs the image) added to *loss, and
+//        the bf16 of the loss gradient to y
 //  CAT   data gradient of a concatenation [up, skip]: channels < up_c are summed
 //        over 2x2 pixels (the upsampling's gradient) and masked into y at half
 //        resolution, the rest go to yf in FP32
@@ -982,7 +983,7 @@ struct UNet {
             ep.cv = cout_real;
             ep.wv = wv;
             ep.hv = hv;
-            ep.inv_count = 1.0 / ((double)B * std::min(wv, W) * std::min(hv, H) * cout_real);
+            ep.inv_count = 1.0 / ((double)B * wv * hv * cout_real);
             ep.loss = d_loss;
             conv3<EPI_MSE, false>(dense(db[0], c(0)), c(0), head().wf, d_p + head().b_off, ep, cout, 0);
         }
@@ -1099,8 +1100,10 @@ int llgmi_ws_create(const llgmi_ws_shape *shape, uint64_t seed, int device, llgm
     ws->device = device;
     try {
         LLGMI_HIP(hipSetDevice(device));
+        // a valid region beyond the plane is the whole plane
         ws->net.reset(new UNet((int)s.batch, (int)s.height, (int)s.width, s.in_channels, s.out_channels,
-                               s.base_channels, (int)s.valid_width, (int)s.valid_height, seed));
+                               s.base_channels, (int)std::min(s.valid_width, s.width),
+                               (int)std::min(s.valid_height, s.height), seed));
     } catch (const Error &e) {
         return ws_fail(e.code, e.what());
     } catch (const std::bad_alloc &) {

@@ -118,6 +118,22 @@ def test_gradient_tile_edges(gpu_lib, batch, height, width, base, out):
             o += k
 
 
+# A valid region beyond the plane is the whole plane, also where the loss's pixel
+# tiles overhang the image on the right (24 = 16 + 8) and below.
+@pytest.mark.parametrize("height,width", [(24, 24), (40, 24), (8, 40)])
+@pytest.mark.parametrize("beyond", [8, 1 << 40])
+def test_valid_region_beyond_the_plane(gpu_lib, height, width, beyond):
+    kw = dict(batch=2, height=height, width=width, out_channels=20, base=16)
+    big = U.Shape(valid_width=width + beyond, valid_height=height + beyond, **kw)
+    net, p, x, t, xd, td = _setup(gpu_lib, big, 31)
+    whole, *_ = _setup(gpu_lib, U.Shape(valid_width=width, valid_height=height, **kw), 31)
+    loss, loss_w = net.loss_grad(xd, td), whole.loss_grad(xd, td)
+    assert abs(loss - loss_w) <= 1e-12 * loss_w   # FP64 sums whose block order is free
+    assert np.array_equal(net.get_grads(), whole.get_grads())
+    loss_o, _, _ = U.loss_and_grad(big, p, x, t, bf16=True)
+    assert abs(loss - loss_o) <= 1e-3 * loss_o
+
+
 def test_training_reduces_loss(gpu_lib):
     """Fit a fixed linear map of the input (a smoothed combination of the
     channels) on one batch: 150 Adam steps cut the loss by 10x."""
