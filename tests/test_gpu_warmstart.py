@@ -134,6 +134,22 @@ def test_valid_region_beyond_the_plane(gpu_lib, height, width, beyond):
     assert abs(loss - loss_o) <= 1e-3 * loss_o
 
 
+@pytest.mark.parametrize("shift", [1, 2, 4])
+def test_targets_on_any_element(gpu_lib, shift):
+    """Targets that start `shift` elements past a 16-byte boundary: the same loss
+    and gradients."""
+    from conftest import DeviceBuffer
+    s = U.Shape(batch=2, height=24, width=24, out_channels=20, base=16, valid_width=22, valid_height=23)
+    net, _, _, t, xd, td = _setup(gpu_lib, s, 33)
+    loss = net.loss_grad(xd, td)
+    g = net.get_grads()
+    off = DeviceBuffer(2 * t.size + 16)
+    off.upload(U.bf16_bits(t), 2 * shift)
+    loss_s = net.loss_grad(xd, off.data_ptr() + 2 * shift)
+    assert abs(loss_s - loss) <= 1e-12 * loss
+    assert np.array_equal(net.get_grads(), g)
+
+
 def test_training_reduces_loss(gpu_lib):
     """Fit a fixed linear map of the input (a smoothed combination of the
     channels) on one batch: 150 Adam steps cut the loss by 10x."""
