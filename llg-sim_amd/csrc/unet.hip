@@ -859,18 +859,25 @@ struct UNet {
         if ((ep.pool || EPI == EPI_CAT) && (hl(l) % 2 || wl(l) % 2)) throw Error(LLGMI_ERR_INVALID, "internal: odd plane");
         // Pixel tile: the largest that gives two blocks to every CU twice over;
         // 16 x 32 reads least per product, but on narrow planes its padding
-        // (columns past the image) costs more than that.  LLGMI_UNET_TILE=0
-        // takes the smallest everywhere.
+        // (columns past the image) costs more than that.  LLGMI_UNET_TILE=8x16 (or
+        // 0), 16x16 or 16x32 takes that tile everywhere (16x32 where it is built).
         auto tiles = [&](int th, int tw) {
             return (int64_t)B * ((hl(l) + th - 1) / th) * ((wl(l) + 16 * tw - 1) / (16 * tw));
         };
         const int64_t groups = co / (16 * nt);
-        const bool wide = nt < 3 && tiles(16, 2) * groups >= 1024 && 10 * 2 * tiles(16, 2) <= 11 * tiles(16, 1);
-        const bool tall = tiles(16, 1) * groups >= 512;
+        bool wide = nt < 3 && tiles(16, 2) * groups >= 1024 && 10 * 2 * tiles(16, 2) <= 11 * tiles(16, 1);
+        bool tall = tiles(16, 1) * groups >= 512;
+        if (const char *e = std::getenv("LLGMI_UNET_TILE")) {
+            const std::string v(e);
+            const bool w32 = v == "16x32";
+            if (w32 || v == "16x16" || v == "8x16" || v[0] == '0') {
+                wide = w32 && nt < 3;
+                tall = w32 || v == "16x16";
+            }
+        }
         auto go = [&](auto ntc) {
             constexpr int NT = decltype(ntc)::value;
-            if (!large_tiles()) launch_conv<8, 1, NT, EPI, RELU>(src, cin, w, bias, ep, co, l);
-            else if (wide) {
+            if (wide) {
                 if constexpr (NT < 3) launch_conv<16, 2, NT, EPI, RELU>(src, cin, w, bias, ep, co, l);
             } else if (tall) launch_conv<16, 1, NT, EPI, RELU>(src, cin, w, bias, ep, co, l);
             else launch_conv<8, 1, NT, EPI, RELU>(src, cin, w, bias, ep, co, l);
@@ -878,10 +885,6 @@ struct UNet {
         if (nt == 3) go(std::integral_constant<int, 3>{});
         else if (nt == 2) go(std::integral_constant<int, 2>{});
         else go(std::integral_constant<int, 1>{});
-    }
-    static bool large_tiles() {
-        const char *e = std::getenv("LLGMI_UNET_TILE");
-        return !(e && e[0] == '0');
     }
     template <int TH, int TW, int NT, int EPI, bool RELU>
     void launch_conv(ConvSrc src, int cin, const uint16_t *w, const float *bias, const ConvEpi &ep, int co, int l) {

@@ -7,7 +7,8 @@
   land on the other side in a few elements: the bars are relative L2 norms,
   forward 1e-5 (measured 6e-8), each layer's gradient 1e-3 (worst measured
   7e-4), all gradients 3e-4 (measured 1.05e-4).  LLGMI_UNET_TILE=0 takes the
-  smallest pixel tile at every level.
+  smallest pixel tile at every level, as planes this small do by themselves;
+  test_pixel_tiles takes each.
 * Adam training on the device reduces the loss of a learnable map.
 * The trained network's potential, written into the multigrid solver as its
   initial phi, reaches the same residual in fewer V-cycles than the zero
@@ -132,6 +133,44 @@ def test_valid_region_beyond_the_plane(gpu_lib, height, width, beyond):
     assert np.array_equal(net.get_grads(), whole.get_grads())
     loss_o, _, _ = U.loss_and_grad(big, p, x, t, bf16=True)
     assert abs(loss - loss_o) <= 1e-3 * loss_o
+
+
+# Every pixel tile of the convolutions on planes whose width is no multiple of 32
+# or 16 and whose height is no multiple of 16, channel tiles of 16, 32 and 48
+# (outputs 20 -> 32, 36 -> 48): all take a sum's terms in one order, so the forward
+# pass and, from it, loss and gradients are equal bit for bit; the smallest one's
+# gradients against the oracle as in test_gradient_tile_edges.
+@pytest.mark.parametrize("batch,height,width,base,out", [
+    (1, 24, 40, 32, 20), (2, 40, 24, 16, 36), (1, 72, 88, 16, 20), (3, 16, 48, 32, 36)])
+def test_pixel_tiles(gpu_lib, batch, height, width, base, out, monkeypatch):
+    from conftest import DeviceBuffer
+    s = U.Shape(batch=batch, height=height, width=width, out_channels=out, base=base, valid_width=width - 1,
+                valid_height=height - 3)
+    net, p, x, t, xd, td = _setup(gpu_lib, s, 41 + height)
+    n = s.batch * s.height * s.width * s.c_pad
+    got = []
+    for tile in ("8x16", "16x16", "16x32"):
+        monkeypatch.setenv("LLGMI_UNET_TILE", tile)
+        yd = DeviceBuffer(4 * n)
+        net.forward(xd, yd)
+        loss = net.loss_grad(xd, td)
+        got.append((yd.download(np.float32, n), loss, net.get_grads()))
+    y_64 = U.forward(s, p, x, bf16=False)[0].reshape(-1)
+    y_b = U.forward(s, p, x, bf16=True)[0].reshape(-1)
+    assert np.linalg.norm(got[0][0] - y_64) <= 2.0 * np.linalg.norm(y_b - y_64)
+    loss_o, g_o, _ = U.loss_and_grad(s, p, x, t, bf16=True)
+    _, g_64, _ = U.loss_and_grad(s, p, x, t, bf16=False)
+    assert abs(got[0][1] - loss_o) <= 1e-3 * loss_o
+    o = 0
+    for li, (ci, co, _) in enumerate(U.layers(s)):
+        for name, k in (("w", 9 * ci * co), ("b", co)):
+            a, b, c = got[0][2][o:o + k], g_o[o:o + k], g_64[o:o + k]
+            assert np.linalg.norm(a - c) <= 2.0 * np.linalg.norm(b - c) + 1e-6 * np.linalg.norm(c), (li, name)
+            o += k
+    for y, loss, g in got[1:]:
+        assert np.array_equal(y, got[0][0])
+        assert abs(loss - got[0][1]) <= 1e-12 * loss   # FP64 sums whose block order is free
+        assert np.array_equal(g, got[0][2])
 
 
 @pytest.mark.parametrize("shift", [1, 2, 4])
@@ -295,8 +334,9 @@ def test_mask_cells_and_unpack_accumulate(gpu_lib):
 
 @pytest.mark.parametrize("h,w", [(240, 264), (256, 264)])
 def test_large_planes_as_accurate_as_bf16_emulation(gpu_lib, h, w):
-    """On planes of 63360 and 67584 pixels (the second runs 64-pixel waves
-    at level 0) the device and the oracle's bf16 emulation each round some
+    """On planes of 63360 and 67584 pixels (16 x 16 pixel tiles in the
+    concatenation's gradient at level 0, 8 x 16 elsewhere) the device and the
+    oracle's bf16 emulation each round some
     activations differently (FP32 vs float64 sums), and through the deep
     levels one such rounding reaches much of the image: the two differ by
     about the bf16 noise itself (measured 3.7e-3 relative, against 6e-3 for
