@@ -2213,7 +2213,12 @@ void MGSolver::smooth(int l, int64_t iters) {
             }
             return;
         }
-        if (rb_fused_ && L.nz >= 3) {
+        // A march takes nz + 4 steps of 0.85 us each however narrow the level is,
+        // because a block owns whole columns; four half-sweep launches take 2.5 us
+        // each and 14.6 us more per million updates.  19 x 19 x 31: 30 us against
+        // 10 us; 76 x 76 x 124: 109 against 31 us; 262 x 262 x 18: 25 against 46 us.
+        const int64_t n = (int64_t)(L.ny - 2) * (L.nz - 2) * ((L.nx - 1) / 2);
+        if (rb_fused_ && L.nz >= 3 && 0.85 * (L.nz + 4) < 4.0 * (2.5 + 14.6e-6 * (double)n)) {
             // pairs of sweeps; the 64 x 32 box where its blocks fill at least
             // half the CUs (its halo is re-read and recomputed least), else 32 x 16
             ensure_pair(L);
@@ -2233,7 +2238,6 @@ void MGSolver::smooth(int l, int64_t iters) {
             }
         }
         // single sweeps: the two half-sweep kernels, in place
-        const int64_t n = (int64_t)(L.ny - 2) * (L.nz - 2) * ((L.nx - 1) / 2);
         for (int64_t it = 0; it < iters; ++it)
             for (int color = 0; color < 2; ++color) {
                 hipLaunchKernelGGL(k_mg_rb, dim3(nblocks(n)), dim3(kNT), 0, stream_, L.phi[L.cur], L.rhs, L.nx,

@@ -86,6 +86,15 @@ def test_mg_smoother_tile_edges(gpu_lib, nx, ny, nvac, pre, post, cycles, op):
     assert rel_err(got, want) <= 1e-12
 
 
+# Both sides of the line between the two-sweep march and the half-sweep launches:
+# wide shallow levels (290 x 202 x 8: tiles of 24 x 8 columns exactly filled, then
+# with remainders) march, narrow deep ones (24 x 18 x 84) do not.
+@pytest.mark.parametrize("nx,ny,nvac,pre,post,cycles", [
+    (286, 198, 3, 2, 2, 2), (288, 196, 3, 4, 2, 2), (20, 14, 40, 2, 2, 3)])
+def test_mg_march_or_half_sweeps(gpu_lib, nx, ny, nvac, pre, post, cycles):
+    test_mg_smoother_tile_edges(gpu_lib, nx, ny, nvac, pre, post, cycles, "rb7_inject_rd")
+
+
 @pytest.mark.parametrize("op", ["rb7_inject_rd", "iso27_tri_galerkin"])
 def test_mg_fp32_context_close_to_oracle(gpu_lib, op):
     from oracle import oracle as O
