@@ -289,8 +289,8 @@ __global__ void __launch_bounds__(kNT) k_mg_rb(double *__restrict__ phi, const d
     phi[id] = po + omega * (pn[0] - po);
 }
 
-// Two red-black SOR sweeps (colours 0, 1, 0, 1) from A into B in one pass over
-// memory.  A block owns a (BX-8) x (BY-8) tile of columns plus a four-cell
+// NS = 2: two red-black SOR sweeps (colours 0, 1, 0, 1) from A into B in one pass
+// over memory.  A block owns a (BX-8) x (BY-8) tile of columns plus a four-cell
 // halo, one thread per pair of columns x = 2c, 2c+1, and marches up z.  The four
 // half-sweeps follow each other through the planes: step s updates colour 0 of
 // the first sweep on plane s and of the second on plane s-3, then (one barrier
@@ -306,19 +306,24 @@ __global__ void __launch_bounds__(kNT) k_mg_rb(double *__restrict__ phi, const d
 // consecutive words.  The march is unrolled over the eight planes of the ring,
 // which makes register and LDS slots constants.
 //
+// NS = 1: one sweep, a two-cell halo, each plane final one step after its first
+// update; for a finest level's odd sweep.
+//
 // Traffic: phi in, rhs in twice (the second time from L2), phi out once for two
 // sweeps.
 // At 524 x 524 x 36: 66 us for two sweeps (3.6 TB/s over phi, rhs and the
 // result once each), against 2 x 98 us for the earlier one-sweep march (which read phi
 // and rhs once per sweep, through a serial division per cell); 80 us without the
 // XCD order.  The 32 x 16 box at 262 x 262 x 18: 25 us against 46 us for four
-// half-sweep launches.
-template <int BX, int BY>
-__global__ void __launch_bounds__(BX *BY / 2) k_mg_rb_sweep2(const double *__restrict__ A, double *__restrict__ B,
+// half-sweep launches.  One sweep at 524 x 524 x 36: 66 us, its two half-sweep
+// launches 164 us.
+template <int BX, int BY, int NS>
+__global__ void __launch_bounds__(BX *BY / 2) k_mg_rb_march(const double *__restrict__ A, double *__restrict__ B,
                                                              const double *__restrict__ rhs, int nx, int ny, int nz,
                                                              double sx, double sy, double sz, ExactDiv denom,
                                                              double omega) {
-    constexpr int HX = BX / 2, TX = BX - 8, TY = BY - 8, PLANE = BX * BY;
+    constexpr int HALO = 2 * NS, LAG = NS == 2 ? 4 : 1;   // LAG: steps from a plane's first update to its last
+    constexpr int HX = BX / 2, TX = BX - 2 * HALO, TY = BY - 2 * HALO, PLANE = BX * BY;
     extern __shared__ unsigned char lds_raw[];
     // a row before and after the planes: rows 0 and BY-1 read (and drop) their neighbours too
     double *lds = reinterpret_cast<double *>(lds_raw) + BX;
@@ -327,7 +332,7 @@ __global__ void __launch_bounds__(BX *BY / 2) k_mg_rb_sweep2(const double *__res
     const int lb = xcd_remap((int)(blockIdx.y * gridDim.x + blockIdx.x), (int)(gridDim.x * gridDim.y));
     const int by = lb / (int)gridDim.x, bx = lb - by * (int)gridDim.x;
     const int i0 = 1 + bx * TX, j0 = 1 + by * TY;
-    const int gi = i0 - 4 + 2 * c, gj = j0 - 4 + y;   // column 2c of the box
+    const int gi = i0 - HALO + 2 * c, gj = j0 - HALO + y;   // column 2c of the box
     // column index 0: the one whose cells are colour 0 on even planes
     const int q = (gi + gj) & 1;
     const bool rowin = gj >= 0 && gj < ny, rowup = y >= 1 && y < BY - 1 && gj >= 1 && gj <= ny - 2;
@@ -367,22 +372,23 @@ __global__ void __launch_bounds__(BX *BY / 2) k_mg_rb_sweep2(const double *__res
         lds[u * PLANE + own[0]] = v[u][0];
         lds[u * PLANE + own[1]] = v[u][1];
     };
-    // one cell each of column a0 on plane k0 and column a1 on plane k1 (ring
-    // slots u0, u1) with right sides r0, r1
+    // one cell each of column a0 on plane k0 and (NS = 2) of column a1 on plane k1
+    // (ring slots u0, u1) with right sides r0, r1
     auto update = [&](int k0, int u0, int a0, double r0, int k1, int u1, int a1, double r1) {
         const int kk[2] = {k0, k1}, uu[2] = {u0, u1}, aa[2] = {a0, a1};
-        double pn[2] = {r0, r1};
+        const double rr[2] = {r0, r1};
+        double pn[NS];
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
+        for (int i = 0; i < NS; ++i) {
             const int u = uu[i], a = aa[i];
             const double *p = lds + u * PLANE;
             const double off = sx * (v[u][1 - a] + p[nbx[a]]) + sy * (p[own[a] - BX] + p[own[a] + BX]) +
                                sz * (v[(u + 7) & 7][a] + v[(u + 1) & 7][a]);
-            pn[i] = off - pn[i];
+            pn[i] = off - rr[i];
         }
         div_by(pn, denom);
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
+        for (int i = 0; i < NS; ++i) {
             const int u = uu[i], a = aa[i];
             if (up[a] && kk[i] >= 1 && kk[i] <= nz - 2) {
                 v[u][a] += omega * (pn[i] - v[u][a]);
@@ -399,24 +405,24 @@ __global__ void __launch_bounds__(BX *BY / 2) k_mg_rb_sweep2(const double *__res
     fetch(2, 2);
     double r[4] = {0.0, 0.0, 0.0, 0.0};   // right sides of a step's four updates
     __syncthreads();
-    for (int s0 = 0; s0 < nz + 4; s0 += 8) {
+    for (int s0 = 0; s0 < nz + LAG; s0 += 8) {
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
             const int s = s0 + u, e = u & 1, o = 1 - e;
-            if (s >= nz + 4) break;
+            if (s >= nz + LAG) break;
             // colour 0 of the first sweep on plane s, of the second on s - 3
             update(s, u, e, r[0], s - 3, (u + 5) & 7, o, r[1]);
             r[0] = fetch_r(s + 1, o);
-            r[1] = fetch_r(s - 2, e);
+            if (NS == 2) r[1] = fetch_r(s - 2, e);
             __syncthreads();
             // colour 1: planes s - 1 and s - 4
             update(s - 1, (u + 7) & 7, e, r[2], s - 4, (u + 4) & 7, o, r[3]);
             r[2] = fetch_r(s, o);
-            r[3] = fetch_r(s - 3, e);
-            if (s >= 4) {   // plane s - 4 is final
+            if (NS == 2) r[3] = fetch_r(s - 3, e);
+            if (s >= LAG) {   // plane s - LAG is final
 #pragma unroll
                 for (int a = 0; a < 2; ++a)
-                    if (out[a]) *const_cast<double *>(cell(B, s - 4, a)) = v[(u + 4) & 7][a];
+                    if (out[a]) *const_cast<double *>(cell(B, s - LAG, a)) = v[(u + 8 - LAG) & 7][a];
             }
             stage((u + 2) & 7);
             fetch(s + 3, (u + 3) & 7);   // the slot of plane s - 5, read for the last time above
@@ -1889,8 +1895,9 @@ MGSolver::MGSolver(const llgmi_grid &g, const llgmi_mg_config &cfg_in, hipStream
         for (const void *k : {(const void *)k_mg_rb_tb<true>, (const void *)k_mg_rb_tb<false>})
             LLGMI_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize,
                                           (int)(sizeof(double) * TB_MAXZ * TBW * TBW)));
-        LLGMI_HIP(hipFuncSetAttribute((const void *)k_mg_rb_sweep2<64, 32>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      (int)(sizeof(double) * (8 * 64 * 32 + 2 * 64))));
+        for (const void *k : {(const void *)k_mg_rb_march<64, 32, 1>, (const void *)k_mg_rb_march<64, 32, 2>})
+            LLGMI_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                          (int)(sizeof(double) * (8 * 64 * 32 + 2 * 64))));
         const size_t n0 = (size_t)px_ * py_ * pz_;
         LLGMI_HIP(hipMalloc((void **)&bc_, sizeof(double) * n0));
         LLGMI_HIP(hipMemsetAsync(bc_, 0, sizeof(double) * n0, stream_));
@@ -2219,25 +2226,32 @@ void MGSolver::smooth(int l, int64_t iters) {
         // 10 us; 76 x 76 x 124: 109 against 31 us; 262 x 262 x 18: 25 against 46 us.
         const int64_t n = (int64_t)(L.ny - 2) * (L.nz - 2) * ((L.nx - 1) / 2);
         if (rb_fused_ && L.nz >= 3 && 0.85 * (L.nz + 4) < 4.0 * (2.5 + 14.6e-6 * (double)n)) {
-            // pairs of sweeps; the 64 x 32 box where its blocks fill at least
-            // half the CUs (its halo is re-read and recomputed least), else 32 x 16
+            // pairs of sweeps, and the finest level's odd one; the 64 x 32 box where
+            // its blocks fill at least half the CUs (its halo is re-read and
+            // recomputed least), else 32 x 16
             ensure_pair(L);
-            auto pair_of = [&](auto bxc, auto byc) {
-                constexpr int BX = decltype(bxc)::value, BY = decltype(byc)::value;
-                const dim3 grid((unsigned)((L.nx - 2 + BX - 9) / (BX - 8)), (unsigned)((L.ny - 2 + BY - 9) / (BY - 8)));
-                hipLaunchKernelGGL((k_mg_rb_sweep2<BX, BY>), grid, dim3(BX * BY / 2), sizeof(double) * (8 * BX * BY + 2 * BX),
-                                   stream_, L.phi[L.cur], L.phi[1 - L.cur], L.rhs, L.nx, L.ny, L.nz, sx, sy, sz, denom,
-                                   cfg_.sor_omega);
-                LLGMI_LAUNCH_CHECK();
-                L.cur = 1 - L.cur;
-            };
             const bool large = (int64_t)((L.nx - 2 + 55) / 56) * ((L.ny - 2 + 23) / 24) >= 128;
-            for (; iters >= 2; iters -= 2) {
-                if (large) pair_of(std::integral_constant<int, 64>{}, std::integral_constant<int, 32>{});
-                else pair_of(std::integral_constant<int, 32>{}, std::integral_constant<int, 16>{});
+            auto march = [&](auto nsc) {
+                auto go = [&](auto bxc, auto byc) {
+                    constexpr int NS = decltype(nsc)::value, BX = decltype(bxc)::value, BY = decltype(byc)::value;
+                    constexpr int TX = BX - 4 * NS, TY = BY - 4 * NS;
+                    const dim3 grid((unsigned)((L.nx - 2 + TX - 1) / TX), (unsigned)((L.ny - 2 + TY - 1) / TY));
+                    hipLaunchKernelGGL((k_mg_rb_march<BX, BY, NS>), grid, dim3(BX * BY / 2),
+                                       sizeof(double) * (8 * BX * BY + 2 * BX), stream_, L.phi[L.cur], L.phi[1 - L.cur],
+                                       L.rhs, L.nx, L.ny, L.nz, sx, sy, sz, denom, cfg_.sor_omega);
+                    LLGMI_LAUNCH_CHECK();
+                    L.cur = 1 - L.cur;
+                };
+                if (large) go(std::integral_constant<int, 64>{}, std::integral_constant<int, 32>{});
+                else go(std::integral_constant<int, 32>{}, std::integral_constant<int, 16>{});
+            };
+            for (; iters >= 2; iters -= 2) march(std::integral_constant<int, 2>{});
+            if (iters == 1 && l == 0) {
+                march(std::integral_constant<int, 1>{});
+                iters = 0;
             }
         }
-        // single sweeps: the two half-sweep kernels, in place
+        // other sweeps: the two half-sweep kernels, in place
         for (int64_t it = 0; it < iters; ++it)
             for (int color = 0; color < 2; ++color) {
                 hipLaunchKernelGGL(k_mg_rb, dim3(nblocks(n)), dim3(kNT), 0, stream_, L.phi[L.cur], L.rhs, L.nx,

@@ -95,6 +95,14 @@ def test_mg_march_or_half_sweeps(gpu_lib, nx, ny, nvac, pre, post, cycles):
     test_mg_smoother_tile_edges(gpu_lib, nx, ny, nvac, pre, post, cycles, "rb7_inject_rd")
 
 
+# The finest level's odd sweep, marched on its own: tiles of 28 x 12 columns exactly
+# filled and with remainders, and the large box's 60 x 28.
+@pytest.mark.parametrize("nx,ny,nvac,pre,post,cycles", [
+    (278, 202, 3, 1, 3, 2), (280, 200, 3, 1, 1, 2), (640, 600, 2, 1, 3, 1)])
+def test_mg_odd_finest_sweep(gpu_lib, nx, ny, nvac, pre, post, cycles):
+    test_mg_smoother_tile_edges(gpu_lib, nx, ny, nvac, pre, post, cycles, "rb7_inject_rd")
+
+
 @pytest.mark.parametrize("op", ["rb7_inject_rd", "iso27_tri_galerkin"])
 def test_mg_fp32_context_close_to_oracle(gpu_lib, op):
     from oracle import oracle as O
