@@ -86,6 +86,29 @@ def test_mg_smoother_tile_edges(gpu_lib, nx, ny, nvac, pre, post, cycles, op):
     assert rel_err(got, want) <= 1e-12
 
 
+# Narrow boxes on the edges of the residual norm's row groups (interior widths 4 to
+# 34) and planes of few and of odd cell counts, with a tolerance: fields, cycles
+# and the last residual.
+@pytest.mark.parametrize("nx,ny", [(1, 7), (3, 500), (5, 41), (11, 30), (13, 200), (27, 9), (29, 33), (31, 100)])
+@pytest.mark.parametrize("op", list(OPS))
+def test_mg_narrow_boxes(gpu_lib, nx, ny, op):
+    from oracle import oracle as O
+    L = gpu_lib
+    cell = (4e-9, 3e-9, 2e-9)
+    lc, oc = _pair(L, O, pad_xy=2, n_vac_z=3, bc=0, warm_start=0, tol_rel=1e-6, v_cycles=1, v_cycles_max=6, **OPS[op])
+    m = _rand_m(nx * ny, nx + ny)
+    want = np.zeros_like(m)
+    omg = O.MG(O.Grid(nx, ny, *cell), oc)
+    omg.add_field(m, want, 8e5)
+    ctx = L.Context(L.Grid2D(nx, ny, *cell), precision=L.F64)
+    ctx.set_mg_config(lc)
+    got = ctx.compute_demag_field_poisson_mg(m, L.Material(ms=8e5, demag=True))
+    assert rel_err(got, want) <= 1e-12
+    st, ost = ctx.mg_last_stats(), omg.stats()
+    assert st["cycles"] == ost["cycles"]
+    assert abs(st["last_residual"] - ost["last_residual"]) <= 1e-12 * ost["rhs_max"]
+
+
 # Both sides of the line between the two-sweep march and the half-sweep launches:
 # wide shallow levels (290 x 202 x 8: tiles of 24 x 8 columns exactly filled, then
 # with remainders) march, narrow deep ones (24 x 18 x 84) do not.
