@@ -2289,7 +2289,13 @@ void MGSolver::smooth(int l, int64_t iters) {
         auto blocks = [&](int T) { return (int64_t)((L.nx - 2 + T - 1) / T) * ((L.ny - 2 + T - 1) / T); };
         int T = 4;
         while (T < WJW - 4 && blocks(T) > 256) T += 2;
-        if ((L.ny - 2 + T - 1) / T <= kGridMax) {
+        // A launch of at most 1024 blocks (four per CU are resident) takes 8.5 us for
+        // (WJW - T) / 2 sweeps, one of more blocks longer in proportion, also where a
+        // narrow level leaves most of a block's columns and planes empty; a sweep of
+        // its own takes 4 us and 7 us more per million cells.  253 x 253 x 9: 4.3 us
+        // a sweep against 8 us; 6 x 270004 x 4: 95 us against 48 us.
+        const double per_sweep = 8.5 * std::max(1.0, (double)blocks(T) / 1024.0) / ((WJW - T) / 2);
+        if (per_sweep < 4.0 + 7e-6 * ((double)L.nx * L.ny * L.nz) && (L.ny - 2 + T - 1) / T <= kGridMax) {
             const dim3 grid((unsigned)((L.nx - 2 + T - 1) / T), (unsigned)((L.ny - 2 + T - 1) / T));
             for (int64_t left = iters; left > 0;) {
                 const int h = (int)std::min<int64_t>(left, (WJW - T) / 2);
