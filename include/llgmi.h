@@ -349,6 +349,7 @@ int llgmi_ws_param_count(llgmi_ws *ws, int64_t *n);
 int llgmi_ws_get_params(llgmi_ws *ws, float *host);
 int llgmi_ws_set_params(llgmi_ws *ws, const float *host);
 int llgmi_ws_get_grads(llgmi_ws *ws, float *host);   /* of the last loss_grad */
+/* x_dev starts on 16 bytes; t_dev and y_dev on any element. */
 int llgmi_ws_forward(llgmi_ws *ws, const uint16_t *x_dev, float *y_dev);
 int llgmi_ws_loss_grad(llgmi_ws *ws, const uint16_t *x_dev, const uint16_t *t_dev, double *loss);
 int llgmi_ws_adam_step(llgmi_ws *ws, double lr);

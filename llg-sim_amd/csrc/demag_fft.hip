@@ -54,9 +54,10 @@ __host__ __device__ constexpr int mini(int a, int b) { return a < b ? a : b; }
 // its full width (64 contiguous bytes: four pairs in FP32, two in FP64; narrower
 // runs store slower, wider ones no faster) and a block at least one wave.  More
 // pairs only make fewer, larger blocks, which leaves small grids on a handful
-// of CUs: at 128 x 64 in FP64 18 pairs per block meant 6 blocks.
-// (now 16): row passes of an RK45 attempt there 10 and 16 us -> 6 and 12 us with
-// radix 8, the attempt 245 -> 165 us; 1024^2 and 2048^2 unchanged.
+// of CUs: at 128 x 64 in FP64 the forward pass has 48 blocks of two pairs, with
+// 18 pairs per block it had 6.  Evaluations (us): 64 x 64 in FP64 17.9 -> 16.0,
+// 256 x 128 padded to 512 x 256 19.4 -> 17.2; 64 x 64 in FP32 15.4 -> 14.4;
+// 1024^2 and 2048^2 unchanged.
 #ifndef LLGMI_ROW_LDS_KB
 #define LLGMI_ROW_LDS_KB 80
 #endif

@@ -1169,7 +1169,8 @@ __device__ __forceinline__ double div_sqrt(double q, double x) {
 // the wave's next node is n + 1 if any lane opened n and skip[n] otherwise.
 // Node, moment and charge loads are wave-uniform.  Each lane sees exactly its
 // own traversal in its own order, and keeps one partial sum per open depth,
-// so its value is the reference's nested recursive sum bit for bit.  The
+// so its value is the reference's nested recursive sum, the same terms in the same
+// order with each quotient within a last-place rounding (div_sqrt).  The
 // partial sums live in LDS, one row of kNT lanes per depth (dynamic LDS of
 // (deepest node depth + 1) rows): indexed by the run-time depth they would
 // otherwise go to per-lane scratch memory.

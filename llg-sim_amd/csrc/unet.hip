@@ -398,7 +398,7 @@ __global__ __launch_bounds__(256, (conv_blocks_per_cu<TW, NT>())) void k_conv3x3
 // `part`, which k_part_sum reduces: no atomics, so gradients do not depend on
 // the order in which blocks finish.  The bias gradient is one more product,
 // with ones, in the blocks of the first ci tile.
-// Bound by the tiles' loads where a layer has few channels (32 x 32: 288
+// Bound by the tiles' loads where a layer has few channels (32 x 32: 72
 // multiply-adds per byte) and by LDS reads elsewhere.  Against one block per tap
 // with 8-byte loads and atomics (and a pass of its own for the bias): 11.3 -> 1.3 ms for the fifteen layers of a
 // 8 x 528 x 528 step (742 -> 84 us per 32 x 32 tiled layer).

@@ -62,11 +62,11 @@ def test_mg_fp64_matches_oracle_with_warm_start(gpu_lib, op, bc):
 
 
 # Smoothers on the edges of their tiles, a few cycles without a tolerance, zero
-# boundary: two-sweep boxes of 32 x 16 (24 x 8 columns) with one, full and
-# remainder tiles, odd sweep counts (the last one in place), coarsest levels of
+# boundary: half-sweep launches with even and odd sweep counts, coarsest levels of
 # nine and fewer planes and of several tiles, a flat box and one that does not
-# coarsen in the plane; 640 x 600 takes the 64 x 32 boxes; 270000 rows exceed
-# the launch grid's second dimension.
+# coarsen in the plane; 640 x 600 marches in 64 x 32 boxes; 270000 rows are more
+# than a launch grid's second dimension takes.  (The march's smaller boxes and its
+# odd sweeps: below.)
 @pytest.mark.parametrize("nx,ny,nvac,pre,post,cycles", [
     (7, 5, 3, 2, 2, 3), (26, 10, 4, 2, 1, 3), (27, 41, 8, 3, 2, 3), (50, 34, 16, 1, 4, 3), (75, 12, 16, 2, 3, 3),
     (131, 90, 5, 2, 2, 2), (640, 600, 2, 2, 2, 1), (1, 270000, 2, 2, 2, 1)])
