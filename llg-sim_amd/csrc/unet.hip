@@ -280,22 +280,25 @@ __global__ __launch_bounds__(256, (conv_blocks_per_cu<TW, NT>())) void k_conv3x3
             // took longer than the convolution); the caller's buffer may start on any
             // element
             const int tid = opaque(threadIdx.x);
-            const bool aligned = (reinterpret_cast<uintptr_t>(ep.tgt) & 15) == 0;
-            for (int e = tid; e < TH * 16 * TW * (CO / 8); e += 256) {
-                const int px = e / (CO / 8), c = (e % (CO / 8)) * 8;
-                const int yy = y0 + px / (16 * TW), xx = x0 + px % (16 * TW);
-                uint4 tv{0u, 0u, 0u, 0u};
-                if (yy < H && xx < W) {
-                    const uint16_t *p = ep.tgt + ((int64_t)(b * H + yy) * W + xx) * cout + co_base + c;
-                    if (aligned) {
-                        tv = *reinterpret_cast<const uint4 *>(p);
-                    } else {
-                        uint16_t *h = reinterpret_cast<uint16_t *>(&tv);
-#pragma unroll
-                        for (int k = 0; k < 8; ++k) h[k] = p[k];
-                    }
+            auto targets = [&](auto load) {
+                for (int e = tid; e < TH * 16 * TW * (CO / 8); e += 256) {
+                    const int px = e / (CO / 8), c = (e % (CO / 8)) * 8;
+                    const int yy = y0 + px / (16 * TW), xx = x0 + px % (16 * TW);
+                    uint4 tv{0u, 0u, 0u, 0u};
+                    if (yy < H && xx < W) tv = load(ep.tgt + ((int64_t)(b * H + yy) * W + xx) * cout + co_base + c);
+                    *reinterpret_cast<uint4 *>(xin + px * OROW + c) = tv;
                 }
-                *reinterpret_cast<uint4 *>(xin + px * OROW + c) = tv;
+            };
+            if ((reinterpret_cast<uintptr_t>(ep.tgt) & 15) == 0) {
+                targets([](const uint16_t *p) { return *reinterpret_cast<const uint4 *>(p); });
+            } else {
+                targets([](const uint16_t *p) {
+                    uint4 tv;
+                    uint16_t *h = reinterpret_cast<uint16_t *>(&tv);
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) h[k] = p[k];
+                    return tv;
+                });
             }
             __syncthreads();
         }
