@@ -1504,9 +1504,9 @@ void DemagFFT<T>::launch_row_inv(T *bd, hipStream_t stream, int rq) {
 // shortens (half the values per thread: an RK45 attempt at 128 x 64 in FP64 takes
 // 163 us against 233 us with radix 16), but its third stage at 256 points costs
 // accuracy: in FP32 the field is 10 to 19 % further from an 80-bit convolution than
-// with radix 16, so FP32 keeps radix 16.  FP64 takes radix 8 up to 512 points, where
-// its twiddles all come from the table and it is the more accurate one
-// (reg_fft_rest).
+// with radix 16, so FP32 keeps radix 16.  FP64 takes radix 8 up to 512 points: at
+// 256 its twiddles all come from the table, which makes it the more accurate one
+// (reg_fft_rest), at 512 the two are equally accurate.
 template <typename T>
 void DemagFFT<T>::autotune(hipStream_t stream, int forced) {
     // LLGMI_FFT_COLPIPE=0|1 forces the one-item-per-block or the persistent

@@ -179,10 +179,10 @@ __device__ __forceinline__ void reg_fft_rest(cpx<T> *v, cpx<T> *seq, int t,
         static_assert(TPS % NS == 0, "butterfly class must not depend on the butterfly");
         // 256 points take 8.4.8 with radix 8 against 16.16: with products for the
         // powers the FP64 field is 3 to 9 % further from an 80-bit convolution, with
-        // every power from the table 5 to 7 % nearer, at the same speed.  Small FP64
-        // grids take radix 8 for its shorter chain, at 256 and 512 points.  (At 1024
-        // points the table's loads cost 4 % of an evaluation of 512 x 512.)
-        constexpr bool ALL = sizeof(T) == 8 && P::R0 == 8 && (LOG2L == 8 || LOG2L == 9);
+        // every power from the table 5 to 7 % nearer, at the same speed.  512 points
+        // and more are as near with products in either radix, and the table's loads
+        // cost them 1 to 4 % of an evaluation (906 x 231: 40.3 -> 40.8 us; 512 x 512).
+        constexpr bool ALL = sizeof(T) == 8 && P::R0 == 8 && LOG2L == 8;
         const TwBase<T, R, ALL> twb = twiddle_load<T, R, ALL>(tw, (t & (NS - 1)) << TWS);
         __syncthreads();  // previous stage's LDS writes are visible
         const cpx<T> *rb = seq + lds_pad(t);
